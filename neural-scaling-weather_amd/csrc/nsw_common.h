@@ -197,20 +197,24 @@ __device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds_addr, uint
                  : "m0");
 }
 
-// Barrier between waves with no fence (a fence would wait for every copy)
-// and compiler-level memory ordering on both sides.
-__device__ __forceinline__ void wg_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
 // s_waitcnt vmcnt(N) only (expcnt / lgkmcnt fields at their "no wait" maxima).
 #define NSW_WAIT_VMCNT(n) \
   __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
 // s_waitcnt lgkmcnt(0) only.
 #define NSW_WAIT_LGKMCNT0() __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14))
 
+// Barrier between waves with no fence (a fence would also wait for every copy
+// and store in flight) and compiler-level memory ordering on both sides.  The
+// wave's own LDS accesses are waited for first: s_barrier by itself does not
+// wait on gfx950 and the compiler adds nothing, so without it a row staged
+// with ds_write could be read by another wave past the barrier before it is
+// written.
+__device__ __forceinline__ void wg_barrier() {
+  asm volatile("" ::: "memory");
+  NSW_WAIT_LGKMCNT0();
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 
 // ------------------------------------------------------- XCD placement ----
 // Workgroups are dispatched round-robin over the 8 XCDs (XCD x receives ids
