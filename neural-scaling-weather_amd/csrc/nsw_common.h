@@ -156,6 +156,12 @@ __device__ __forceinline__ float rows4_max(float x) {
   return fmaxf(c, d);
 }
 
+// Maximum over the four lanes of a quad, on every lane.
+__device__ __forceinline__ float quad_max(float x) {
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, false)));
+  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, false)));
+}
+
 // ------------------------------------------- direct-to-LDS copies, waits ----
 // Buffer resource (V#) over a whole tensor: raw buffer, stride 0, 32-bit
 // byte offsets, num_records = bytes, dword 3 = 0x00020000 (the gfx9 raw
@@ -202,6 +208,16 @@ __device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds_addr, uint
   __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | ((((n) >> 4) & 3) << 14))
 // s_waitcnt lgkmcnt(0) only.
 #define NSW_WAIT_LGKMCNT0() __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14))
+
+// Waits until at most N of this wave's copies are in flight; its LDS reads of
+// what they wrote stay behind the wait (the copies are asm that the compiler
+// does not see as writes).
+template <int N = 0>
+__device__ __forceinline__ void wait_copies() {
+  asm volatile("" ::: "memory");
+  NSW_WAIT_VMCNT(N);
+  asm volatile("" ::: "memory");
+}
 
 // Barrier between waves with no fence (a fence would also wait for every copy
 // and store in flight) and compiler-level memory ordering on both sides.  The
