@@ -1,10 +1,47 @@
 // MFMA GEMM y[M,N] = epilogue(x[M,K] . w[N,K]^T): the C ABI and the choice of
 // the tile (kernel: nsw_gemm_kernel.h).
 #include <algorithm>
+#include <cmath>
 
 #include "nsw_gemm_tiles.h"
 
 namespace nsw {
+
+// Tile size by estimated time: rounds of workgroups over the chip's slots, a
+// round of K costing fa + fb K us when every slot is taken and pa + pb K while
+// at most the share f0 of the slots is (between them linear).  The constants
+// are fits to measured times (M 648 - 129600, N 32 - 4096, K 32 - 2048, bias
+// epilogue, within ~15%); 256 x 256 stays unless a smaller tile is estimated 7%
+// faster, since its epilogues are the tuned ones.  Measured, us, 256 x 256 /
+// 128 x 128 / 64 x 128:
+//   bf16   648 x  512, K  128:  7.8 /  4.7 /  3.8    16200 x  192, K  768: 17.7 / 11.2 / 10.6
+//   bf16  8100 x 1024, K 1024: 24.8 / 20.5 / 27.6    64800 x  512, K  512: 41.1 / 46.4 / 55.4
+//   fp32   648 x  128, K  512: 41.0 / 22.2 / 17.2    16200 x  192, K  768: 57.3 / 35.0 / 33.8
+//   fp32 129600 x 128, K   32: 27.1 / 17.3 / 17.9    32400 x  512, K  512: 62.2 / 76.5 / 90.0
+struct TileCost {
+  int64_t bm, bn;
+  double slots, fa, fb, pa, pb, f0;
+  double us(int64_t M, int64_t N, int64_t K) const {
+    const double t = (double)(((M + bm - 1) / bm) * ((N + bn - 1) / bn)) / slots;
+    const double r = std::floor(t), f = t - r, full = fa + fb * (double)K, part = pa + pb * (double)K;
+    return r * full + (f > 0 ? part + std::max(0.0, f - f0) / (1 - f0) * (full - part) : 0);
+  }
+};
+
+template <typename T, int EPI>
+static TileSize pick_tile(int64_t M, int64_t N, int64_t K, const EpiArgs& ea) {
+  using C = TileChoice<T, EPI>;
+  constexpr bool F32 = sizeof(T) == 4;
+  if (EPI == EPI_UNPATCH && ea.img_p == 16) return TILE_BIG;   // a patch of one channel is 256 columns
+  constexpr TileCost big = F32 ? TileCost{256, 256, 256, 18, .0795, 9.5, .0605, 0} : TileCost{256, 256, 256, 8.5, .0234, 5.5, .015, 0};
+  constexpr TileCost mid = F32 ? TileCost{C::Mid::BM, C::Mid::BN, 512, 8, .0537, 6, .0324, .4}
+                               : TileCost{C::Mid::BM, C::Mid::BN, 512, 4.5, .0152, 3.6, .0088, .4};
+  constexpr TileCost small = F32 ? TileCost{C::Small::BM, C::Small::BN, 768, 5, .051, 4.3, .0252, .3}
+                                 : TileCost{C::Small::BM, C::Small::BN, 512, 2.3, .0099, 3.1, .0062, .4};
+  const double b = big.us(M, N, K), m = mid.us(M, N, K), s = small.us(M, N, K);
+  if (std::min(m, s) > 0.93 * b) return TILE_BIG;
+  return s < m ? TILE_SMALL : TILE_MID;
+}
 
 template <typename T, int EPI, int PRE>
 static int launch_gemm(const void* x, const void* w, void* y, int64_t M, int64_t N, int64_t K, const EpiArgs& ea,
@@ -26,7 +63,12 @@ static int launch_gemm(const void* x, const void* w, void* y, int64_t M, int64_t
     // than the other height on its shape)
     if (eg.group_m == 0) eg.group_m = (int)std::max<int64_t>(8, std::min<int64_t>(32, 128 / ((N + 255) / 256)));
   }
-  return launch_tile<T, EPI, PRE, BigTile>(x, w, y, M, N, K, eg, st, what);
+  using C = TileChoice<T, EPI>;
+  switch (pick_tile<T, EPI>(M, N, K, ea)) {
+    case TILE_BIG: return launch_tile<T, EPI, PRE, BigTile>(x, w, y, M, N, K, eg, st, what);
+    case TILE_MID: return launch_tile<T, EPI, PRE, typename C::Mid>(x, w, y, M, N, K, eg, st, what);
+    default: return launch_tile<T, EPI, PRE, typename C::Small>(x, w, y, M, N, K, eg, st, what);
+  }
 }
 
 template <int EPI, int PRE = PRE_NONE>

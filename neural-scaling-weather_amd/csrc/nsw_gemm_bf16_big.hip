@@ -2,7 +2,7 @@
 #include "nsw_gemm_kernel.h"
 
 #define NSW_GEMM_T bf16
-#define NSW_GEMM_TILE BigTile
+#define NSW_GEMM_SIZE Big
 
 namespace nsw {
 NSW_GEMM_FORMS(NSW_GEMM_INSTANCE)

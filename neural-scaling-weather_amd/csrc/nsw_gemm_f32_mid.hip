@@ -1,0 +1,10 @@
+// GEMM instances: fp32, mid tiles.
+#undef NSW_GEMM_STAMPS
+#include "nsw_gemm_kernel.h"
+
+#define NSW_GEMM_T float
+#define NSW_GEMM_SIZE Mid
+
+namespace nsw {
+NSW_GEMM_FORMS(NSW_GEMM_INSTANCE)
+}  // namespace nsw

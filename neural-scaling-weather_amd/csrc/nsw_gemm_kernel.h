@@ -97,8 +97,8 @@ template <typename T, class TC> struct Stg {
   static constexpr int ROWS = TC::BM * STRIDE + PRMB <= TC::LDS ? TC::BM : TC::BM / 2;
   static constexpr int PASSES = TC::BM / ROWS;
   static constexpr int BYTES = ROWS * STRIDE;
-  // operand ring: x in 3 and w in 2 slots (mainloop_256), NST stages (bf16), two (fp32)
-  static constexpr int RING = is_main256<T, TC> ? 5 * 256 * ROWB : (sizeof(T) == 4 ? 2 : TC::NST) * TC::SLOT;
+  // operand ring: x in 3 and w in 2 slots (mainloop_256), else NST stages
+  static constexpr int RING = is_main256<T, TC> ? 5 * 256 * ROWB : TC::NST * TC::SLOT;
   static constexpr int PARAM_LDS = BYTES;
   static constexpr int SMEM = RING > BYTES + PRMB ? RING : BYTES + PRMB;
   static_assert(SMEM <= TC::LDS, "LDS use exceeds the workgroup's share");
@@ -396,6 +396,50 @@ template <typename T, class TC> struct StageCopy {
   }
 };
 
+// bf16 main loop with a ring of NST stages, one barrier per stage: at the top
+// of stage s a wave waits for its copies of stage s, and past the barrier
+// (every wave's copies have landed, and every wave is done reading stage s -
+// 1) it issues the copies of stage s + NST - 1 into the slot of stage s - 1.
+template <class TC>
+__device__ __forceinline__ void mainloop_ring(char* smem, const bf16* __restrict__ X, const bf16* __restrict__ Wt, int M,
+                                              int N, int K, int m0, int n0, f32x4 (&acc)[TC::NB][TC::MB], int wave,
+                                              int lane) {
+  constexpr int NB = TC::NB, MB = TC::MB, NST = TC::NST;
+  using Copy = StageCopy<bf16, TC>;
+  Copy cp;
+  cp.init(smem, X, Wt, M, N, K, m0, n0, wave, lane);
+  const int nst = cp.nst;
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nst) cp.copy(s, s, 0, Copy::NC);
+  const int frow = lane & 15, fg = lane >> 4;
+  const int xrow = (wave / TC::WGN) * TC::WTM + frow;             // x rows of this wave (B operand)
+  const int wrow = TC::BM + (wave % TC::WGN) * TC::WTN + frow;    // w rows of this wave (A operand)
+  int slot = 0;
+  for (int s = 0; s < nst; ++s) {
+    // copies of the up to NST - 2 stages after s may stay in flight
+    if (nst - 1 - s >= NST - 2) NSW_WAIT_VMCNT((NST - 2) * Copy::NC);
+    else NSW_WAIT_VMCNT(0);
+    wg_barrier();
+    if (s + NST - 1 < nst) cp.copy(s + NST - 1, slot == 0 ? NST - 1 : slot - 1, 0, Copy::NC);
+    const char* st = smem + slot * TC::SLOT;
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      if (sub == 1 && (cp.nk & 1) != 0 && s == nst - 1) break;   // the unused half of the last stage
+      bf16x8 fa[NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) fa[nb] = __builtin_bit_cast(bf16x8, lds_frag(st, wrow + nb * 16, 4 * sub + fg));
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        const bf16x8 fb = __builtin_bit_cast(bf16x8, lds_frag(st, xrow + mb * 16, 4 * sub + fg));
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) mfma_bf16(acc[nb][mb], fa[nb], fb);
+      }
+    }
+    slot = slot + 1 == NST ? 0 : slot + 1;
+  }
+}
+
 // fp32 main loop on two fp16 parts of each operand (rows scaled by powers of
 // two), three products.  A stage is 32 k: one step of the 16-bit matrix
 // instructions, lane group g taking k 4g..4g+3 and 16+4g..+3 of both operands.
@@ -406,10 +450,10 @@ template <typename T, class TC> struct StageCopy {
 // wave that reads it: the wave that copied 16 stage rows splits them in place,
 // the h parts into the chunk of k 4c.. and the l parts into that of 16+4c...
 //
-// Two slots.  In stage s the wave splits its rows of stage s + 1 under the
-// MFMAs before row block BARB; the stage's one barrier stands there, once
+// A ring of NST slots.  In stage s the wave splits its rows of stage s + 1 under
+// the MFMAs before row block BARB; the stage's one barrier stands there, once
 // every fragment of the stage is in registers: past it the next stage's first
-// fragments are read, and the copies of stage s + 2 start into the slot just
+// fragments are read, and the copies of stage s + NST start into the slot just
 // read.  Issued in one go the copies hold every wave for the ~1000 cycles that
 // the CU's address path takes for 64 KB, so they are spread, and they carry no
 // condition (past the end they re-read the last stage into a slot whose values
@@ -425,7 +469,7 @@ template <class TC>
 __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restrict__ X, const float* __restrict__ Wt,
                                                 int M, int N, int K, int m0, int n0, f32x4 (&acc)[TC::NB][TC::MB],
                                                 int wave, int lane) {
-  constexpr int NB = TC::NB, MB = TC::MB;
+  constexpr int NB = TC::NB, MB = TC::MB, NST = TC::NST;
   constexpr int BARB = MB > 2 ? MB - 2 : 1;      // row block before which the barrier stands
   using Copy = StageCopy<float, TC>;
   constexpr int NC = Copy::NC, NU = NC / 2;      // copies, 16-row units to split
@@ -435,8 +479,13 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
   Copy cp;
   cp.init(smem, X, Wt, M, N, K, m0, n0, wave, lane);
   const int nst = cp.nst;
-  cp.copy(0, 0, 0, NC);
-  cp.copy(nst > 1 ? 1 : 0, 1, 0, NC1);
+  // deep rings copy stages that exist only (short sums end before their ring
+  // is full; the branch matters less than draining copies nobody needs)
+  constexpr bool COND = NST > 2;
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (!COND || s < nst) cp.copy(s < nst ? s : nst - 1, s, 0, NC);
+  if (!COND || NST - 1 < nst) cp.copy(NST - 1 < nst ? NST - 1 : nst - 1, NST - 1, 0, NC1);
   // this lane's row of a unit and its chunk pair (c, c + 4): any 16 lanes
   // cover four rows whose pairs lie in distinct banks
   const int li = lane >> 2, lc = lane & 3;
@@ -444,7 +493,8 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
   const int uoff = urow * ROWB + (lc ^ row_swizzle(urow)) * 16;   // chunk c; chunk c + 4 is at ^ 64
   auto unit = [&](int u) { return (u < Copy::CX / 2 ? 0 : TC::BM * ROWB) + cp.row(2 * u) * ROWB + uoff; };
   float sc[NU];
-  wait_copies<NC1>();
+  if (!COND || NST <= nst) wait_copies<(NST - 2) * NC + NC1>();
+  else wait_copies();
 #pragma unroll
   for (int u = 0; u < NU; ++u) {
     char* p = smem + unit(u);
@@ -487,11 +537,14 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
   for (int nb = 0; nb < NB; ++nb) load(smem, wrow + nb * 16, ws[nb]);
   load(smem, xrow, xs[0]);
   load(smem, xrow + 16, xs[1]);
+  int slot = 0;
   for (int s = 0; s < nst; ++s) {
-    char* st = smem + (s & 1) * TC::SLOT;
-    char* sn = smem + ((s + 1) & 1) * TC::SLOT;
-    const int c1 = s + 1 < nst ? s + 1 : nst - 1, c2 = s + 2 < nst ? s + 2 : nst - 1;
-    cp.copy(c1, (s + 1) & 1, NC1, NC);
+    const int nslot = slot + 1 == NST ? 0 : slot + 1, pslot = slot == 0 ? NST - 1 : slot - 1;
+    char* st = smem + slot * TC::SLOT;
+    char* sn = smem + nslot * TC::SLOT;
+    // the rest of stage s + NST - 1 here, most of stage s + NST past the barrier
+    const int c1 = s + NST - 1, c2 = s + NST;
+    if (!COND || c1 < nst) cp.copy(c1 < nst ? c1 : nst - 1, pslot, NC1, NC);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       if (mb == BARB) {
@@ -501,11 +554,14 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
       }
       if (mb >= BARB) {
         constexpr int L = MB - BARB;                 // row blocks past the barrier
-        cp.copy(c2, s & 1, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
+        if (!COND || c2 < nst) cp.copy(c2 < nst ? c2 : nst - 1, slot, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
       }
       if (mb + 2 < MB) load(st, xrow + (mb + 2) * 16, xs[(mb + 2) % 3]);
       // the units of the next stage, split ahead of the barrier
-      if (mb == SPLB) wait_copies();
+      if (mb == SPLB) {
+        if (!COND || c1 < nst) wait_copies<(NST - 2) * NC>();
+        else wait_copies();
+      }
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         if (mb != SPLB + u * (BARB - SPLB) / NU) continue;
@@ -531,6 +587,7 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 2; ++i) ws[nb][i] = wn[nb][i];
+    slot = nslot;
   }
   wait_copies();       // those past the last stage
   wg_barrier();        // the ring is no longer read
@@ -799,6 +856,8 @@ __global__ __launch_bounds__(TC::NW * 64, TC::MINW) void gemm_kernel(const T* __
     if constexpr (is_main256<T, TC>) {
       if (wave < 4) mainloop_256<T, 8>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0, rev, ts[1]);
       else mainloop_256<T, 0>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0, rev, ts[1]);
+    } else if constexpr (sizeof(T) == 2) {
+      mainloop_ring<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
     } else {
       bool three = K < SPLIT2_MIN_K;
       if (!three) {
@@ -1234,5 +1293,5 @@ int launch_tile(const void* x, const void* w, void* y, int64_t M, int64_t N, int
 }  // namespace nsw
 
 #define NSW_GEMM_INSTANCE(EPI, PRE)                                                                          \
-  template int launch_tile<NSW_GEMM_T, EPI, PRE, NSW_GEMM_TILE>(                \
+  template int launch_tile<NSW_GEMM_T, EPI, PRE, TileChoice<NSW_GEMM_T, EPI>::NSW_GEMM_SIZE>(                \
       const void*, const void*, void*, int64_t, int64_t, int64_t, const EpiArgs&, hipStream_t, const char*);

@@ -25,6 +25,33 @@ struct TileCfg {
 };
 // 256 x 256, one workgroup of 8 wavefronts per CU: the large problems
 using BigTile = TileCfg<2, 4, 8, 2, 160 * 1024>;
+// Smaller tiles of 4 wavefronts, two or three workgroups per CU, for problems
+// that leave CUs idle at 256 x 256 (pick_tile).  The Row tiles are 256 columns
+// wide (512 bytes of bf16 row, the unit of the row sums of squares).  Deeper
+// rings with one workgroup per CU were slower at every size: with few
+// wavefronts a stage's time is its chain of barrier, LDS reads and issue, not
+// the copies' latency; 8 wavefronts of half the rows per 128 x 128 tile
+// measured the same.
+using MidTile = TileCfg<2, 2, 4, 2, 80 * 1024>;         // 128 x 128
+using MidRowTile = TileCfg<1, 4, 4, 2, 80 * 1024>;      // 64 x 256
+using SmallTile = TileCfg<2, 2, 2, 3, 80 * 1024>;       // 64 x 128, bf16
+using SmallRowTile = TileCfg<1, 4, 2, 2, 80 * 1024>;    // 32 x 256, bf16
+using SmallF32Tile = TileCfg<2, 2, 2, 2, 53 * 1024>;    // 64 x 128, fp32
+
+// Epilogues that store rows through a map or write row sums of squares: in
+// bf16 these take the Row tiles (a 512-byte part of a row lies in one tile).
+constexpr bool row_epi(int epi) {
+  return epi == EPI_SCATTER_RESIDUAL || epi == EPI_REMAP_RESIDUAL || epi == EPI_WINDOW_RESIDUAL ||
+         epi == EPI_RES_SUMSQ || epi == EPI_TOKEN_RESIDUAL;
+}
+
+enum TileSize { TILE_BIG, TILE_MID, TILE_SMALL };
+template <typename T, int EPI> struct TileChoice {
+  static constexpr bool ROW = sizeof(T) == 2 && row_epi(EPI);
+  using Big = BigTile;
+  using Mid = std::conditional_t<ROW, MidRowTile, MidTile>;
+  using Small = std::conditional_t<sizeof(T) == 4, SmallF32Tile, std::conditional_t<ROW, SmallRowTile, SmallTile>>;
+};
 
 // Launches gemm_kernel<T, EPI, PRE, TC> (shapes and alignment checked by the
 // caller).  Defined in nsw_gemm_kernel.h, instantiated by one source per dtype

@@ -93,3 +93,50 @@ def test_split_gemm_non_finite(K):
     keep[[7, 9, 11, 13]] = False
     want = x[keep].double() @ w.double().t()
     assert ((y[keep].double() - want).abs() <= U * (K / 8 + 4) * want).all()
+
+
+# Shapes on both sides of the tile rule (few rows: 64- / 32-row tiles; some
+# hundreds: 128- / 64-row tiles; then 256), with rows and columns that end
+# inside a tile, odd k stages, and every kind of write-out: plain, GELU,
+# residual, the head norm, window maps with row sums, the head's image.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,W,C", [(9, 18, 96), (27, 54, 128), (45, 108, 192), (90, 90, 512)])
+def test_tile_sizes(dtype, H, W, C):
+    g = torch.Generator(device=_dev()).manual_seed(H + C)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=_dev()).to(dtype)
+    M, hd = H * W, 32
+    x, b, r = rnd(M, C), rnd(C), rnd(M, C)
+    w = (0.05 * torch.randn(C, C, generator=g, device=_dev())).to(dtype)
+    w3, b3 = (0.05 * torch.randn(3 * C, C, generator=g, device=_dev())).to(dtype), rnd(3 * C)
+    qn, kn = rnd(hd), rnd(hd)
+    d = lambda t: t.double()
+    tol = 1e-6 if dtype == torch.float32 else 5e-3     # K <= 512: U sqrt(K) < 1e-6; bf16 store 2^-8 / sqrt(3)
+
+    def close(y, want):
+        e = (d(y) - want).norm() / want.norm()
+        assert e < tol, float(e)
+
+    base = d(x) @ d(w).t()
+    close(_linear(x, w), base)
+    close(nsw.ops.linear(x, w, b, r), base + d(b) + d(r))
+    close(nsw.ops.linear(x, w, b, None, epilogue=_lib.NSW_EPI_BIAS_GELU), torch.nn.functional.gelu(base + d(b)))
+    eps = 1e-5
+    qkv = (d(x) @ d(w3).t() + d(b3)).view(M, 3, C // hd, hd)
+    n = qkv * torch.rsqrt(qkv.pow(2).mean(-1, keepdim=True) + eps)
+    want = torch.stack([n[:, 0] * d(qn), n[:, 1] * d(kn), qkv[:, 2]], 1).view(M, 3 * C)
+    close(nsw.ops.qkv_projection(x, w3, b3, qn, kn, C // hd, eps), want)
+    # window rows to the next block's window order, with row sums
+    y, ss = nsw.ops.linear_remap_residual(x, w, b, r, 2, image=(1, 1, H, W), window_size=(9, 18), shift_size=(0, 0),
+                                          next_shift=(4, 9))
+    rows = torch.arange(M, device=_dev()).view(H // 9, W // 18, 9, 18).permute(0, 2, 1, 3).reshape(H, W)
+    nxt = torch.roll(rows, (-4, -9), (0, 1)).view(H // 9, 9, W // 18, 18).permute(0, 2, 1, 3).reshape(-1)
+    want = (base + d(b) + d(r))[nxt]
+    close(y, want)
+    assert torch.allclose(ss.double().sum(1), d(y).pow(2).sum(1), rtol=1e-5)
+    # tokens to image planes
+    for p in (2, 16):
+        ch = 5 * 4 // p if p < 16 else 1
+        wh = (0.05 * torch.randn(ch * p * p, C, generator=g, device=_dev())).to(dtype)
+        img = nsw.ops.head_unpatchify(x, wh, 1, ch, H * p, W * p, p)
+        want = (d(x) @ d(wh).t()).view(H, W, ch, p, p).permute(2, 0, 3, 1, 4).reshape(1, 1, ch, H * p, W * p)
+        close(img, want)
