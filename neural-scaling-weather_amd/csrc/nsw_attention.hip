@@ -26,10 +26,15 @@
 // Workgroup ids are remapped so that the heads of a window share one XCD.
 // Padding keys get -inf logits; no FLOPs are counted for them.
 //
-// Generic path (attn_scalar_kernel, fp32 and any head dim): one thread per
-// query, online softmax over 64-key chunks staged in LDS, fp32 throughout.
+// fp32 (attn_f32_mfma_kernel): any head dim and mask, windows of up to 384
+// tokens, on the fp32 matrix instructions.
+//
+// Generic path (attn_scalar_kernel: larger windows, bf16 at other head dims):
+// one thread per query, online softmax over 64-key chunks staged in LDS, fp32
+// throughout.
 #include "nsw_common.h"
 
+#include <cmath>
 #include <utility>
 
 namespace nsw {
@@ -619,165 +624,228 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------- fp32 MFMA ----
-// fp32 (the reference's inference precision), head dim 64, 9 x 18 windows,
-// shift mask from indices or none: one 512-thread workgroup per (window,
-// head).  K and V rows (256 B of fp32) are copied straight into LDS with
-// their 16-byte chunks XOR-swizzled by row: K chunk c of row r at
-// c ^ (r & 15) (a fragment read, 16 rows x one chunk, covers every bank), V
-// chunk c at c ^ (((r >> 2) & 3) << 2) (the rows 16kb + 4g + r' that lane
-// groups g read in one PV step fall in different 64-byte bank groups).  With
-// v_mfma_f32_16x16x4_f32:
-//   S^T = K Q^T: four MFMAs per 16-byte K fragment (instruction e takes head
-//     dims 16s + 4g + e from lane group g), so lane (i, g) holds the logits of
-//     query i for keys 16kb + 4g + r as in the bf16 kernels, and the mask and
-//     exp2-domain softmax are theirs (probabilities stay fp32);
+// fp32 for every head dim, windows of up to 384 tokens, shift mask from indices,
+// a mask tensor or none.  One workgroup of NW waves per (window, head); wave w
+// owns the query blocks w, w + NW, w + 2 NW.  K and V pass through LDS in chunks
+// of CKB 16-key blocks (at most 48 KB, so that three workgroups share a CU);
+// each query block keeps its output, row maximum and row sum in registers from
+// chunk to chunk (online softmax).  v_mfma_f32_16x16x4_f32:
+//   S^T = K Q^T: lane group g supplies head dims 16s + 4g + e (hd / 4 per group
+//     below 16) of key row i (A) and query i (B), so lane (i, g) holds the
+//     logits of query i for keys 16kb + 4g + r;
 //   O^T = V^T P^T: for key step (kb, r) lane (i, g) supplies V[16kb + 4g + r]
-//     [16db + i] (A) and its own probability for key 16kb + 4g + r (B);
-//   row sums of P on the VALU (lane sums, then across the four lane groups).
-// Lane (i, g) ends with O[query i][16db + 4g .. +3]: one 16-byte store per
-// dim block.  The eight waves (two per SIMD) take query blocks w and w + 8.
-// Key rows past L are zero-filled by the copies' range check (V) or masked to
-// -inf (K).
-template <int NKB>
-__global__ __launch_bounds__(512, 1) void attn_f32_kernel(AttnArgs a, int nitems) {
-  constexpr int HD = 64;
-  constexpr int KR = NKB * 16;                  // rows of K and of V in LDS
-  constexpr int PART = KR * HD * 4;
-  constexpr int NW = 8;
-  constexpr int RG = KR / 4;                    // 4-row copies per part
-  static_assert((2 * RG) % NW == 0, "copies split evenly over the waves");
-  constexpr int NDMA = 2 * RG / NW;
-  constexpr int QPW = (NKB + NW - 1) / NW;
-  constexpr int NS = HD / 16, NDB = HD / 16, NCLS = (KR + 63) / 64;
-  constexpr float LOG2E = 1.4426950408889634f;
-  __shared__ __attribute__((aligned(1024))) char smem[2 * PART];
+//     [16db + i] (A) and its own probability (B); below head dim 16 the lanes
+//     past the head repeat its dims and are not stored (head dim 4 on the VALU
+//     instead spilled).
+// Rows are padded by 16 bytes in LDS: fragment reads (16 rows, one chunk) and the
+// V reads (4 rows 4 apart, 64 bytes each) then cover every bank once.
+// Probabilities, sums and outputs stay fp32.  Bound by the fp32 matrix rate and
+// the softmax's VALU work.  Measured, us, before (head dim 64, 9 x 18, no mask
+// tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
+// others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
+// 540; the same 200 x 8 with a mask tensor: 830 / 214; 100 x 6 of 32: 132 / 47;
+// 400 windows of 324, 8 heads of 4: 630 / 212; 100 x 8 of 64: 1226 / 293.
+template <int HD> struct AttnF32 {
+  static constexpr int STR = HD == 4 ? 16 : HD * 4 + 16;       // bytes per K / V row
+  static constexpr int CKB = HD <= 32 ? 11 : HD == 64 ? 6 : 3; // 16-key blocks per chunk
+  static constexpr int ROWS = CKB * 16;
+  static constexpr int NDB = HD >= 16 ? HD / 16 : 1;           // 16-wide output blocks
+  static constexpr int QN = HD / 4;                            // head dims per lane group
+};
 
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
+template <int HD, int NW, bool MT>
+__global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kernel(AttnArgs a) {
+  using F = AttnF32<HD>;
+  constexpr int STR = F::STR, CKB = F::CKB, ROWS = F::ROWS, NDB = F::NDB, QN = F::QN;
+  constexpr int QPW = 3;
+  constexpr float LOG2E = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(16))) char Ks[ROWS * STR];
+  __shared__ __attribute__((aligned(16))) char Vs[ROWS * STR];
+  __shared__ __attribute__((aligned(4))) unsigned char cls[ROWS];   // shift-mask class of the chunk's keys
+
+  const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int fr = lane & 15, fg = lane >> 4;
-  const int L = a.L, C = a.C;
-  const uint32_t ld = 3u * (uint32_t)C;
-  const int item = xcd_remap((int)blockIdx.x, (int)gridDim.x);
-  const int win = item / a.heads, head = item - win * a.heads;
-  const uint32_t qkv_bytes = (uint32_t)((uint64_t)nitems / a.heads * L * ld * 4u);
-  const u32x4 rq = uniform_rsrc(a.qkv, qkv_bytes);
+  const int L = a.L;
+  const int64_t ld = 3 * (int64_t)a.C;
+  const uint32_t item = (uint32_t)xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const uint32_t win = a.dheads.div(item);
+  const int head = (int)(item - win * (uint32_t)a.heads);
+  const float* base = (const float*)a.qkv + (int64_t)win * L * ld + head * HD;
+  const bool shifted = !MT && window_in_last_band(a, win);
+  const int thr = shifted ? (a.g.ws0 - a.g.s0) * a.g.ws1 : 0, wa = shifted ? a.g.wa : 1;
+  const int nqb = (L + 15) / 16;
 
-  // K rows to [0, PART), V rows to [PART, 2 PART)
-  const uint32_t sbase = (uint32_t)(uintptr_t)smem;
-  const uint32_t soff = ((uint32_t)win * (uint32_t)L * ld + (uint32_t)head * HD) * 4u;
+  f32x4 O[QPW][NDB];
+  float mx[QPW], l[QPW];
 #pragma unroll
-  for (int j = 0; j < NDMA; ++j) {
-    const int d = wave * NDMA + j;
-    const int part = d / RG, rg = d - part * RG;
-    const int row = rg * 4 + lane / 16;
-    const int sw = part == 0 ? (row & 15) : (((row >> 2) & 3) << 2);
-    const int c = (lane % 16) ^ sw;
-    const uint32_t voff = part == 1 && row >= L
-                              ? qkv_bytes
-                              : ((uint32_t)row * ld + (uint32_t)(part + 1) * (uint32_t)C) * 4u + (uint32_t)c * 16u;
-    dma16(rq, sbase + (uint32_t)(part * PART + rg * 1024), voff, soff);
+  for (int i = 0; i < QPW; ++i) {
+    mx[i] = -INFINITY;
+    l[i] = 0.f;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) O[i][db] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  const bool shifted = window_in_last_band(a, win);
-  uint64_t cls[NCLS];
-  {
-    const int thr = shifted ? (a.g.ws0 - a.g.s0) * a.g.ws1 : 0;
-    const int wa = shifted ? a.g.wa : 1;
+  for (int k0 = 0; k0 < L; k0 += ROWS) {
+    __syncthreads();
+    constexpr int CPR = HD / 4;                  // 16-byte chunks per row
+    for (int idx = tid; idx < ROWS * CPR; idx += NW * 64) {
+      const int row = idx / CPR, c = idx - row * CPR;
+      const int key = k0 + row;
+      f32x4 kv = {0.f, 0.f, 0.f, 0.f}, vv = kv;
+      if (key < L) {
+        const float* p = base + key * ld + 4 * c;
+        kv = *reinterpret_cast<const f32x4*>(p + a.C);
+        vv = *reinterpret_cast<const f32x4*>(p + 2 * a.C);
+      }
+      *reinterpret_cast<f32x4*>(Ks + row * STR + c * 16) = kv;
+      *reinterpret_cast<f32x4*>(Vs + row * STR + c * 16) = vv;
+    }
+    if (shifted)
+      for (int row = tid; row < ROWS; row += NW * 64) cls[row] = (k0 + row) % wa >= thr ? 1 : 0;
+    __syncthreads();
 #pragma unroll
-    for (int w = 0; w < NCLS; ++w) {
-      const int key = 64 * w + lane;
-      cls[w] = __ballot(shifted && key < L && (key % wa) >= thr);
+    for (int i = 0; i < QPW; ++i) {
+      const int qb = wave + NW * i;
+      if (qb >= nqb) break;
+      // an offset the compiler cannot see through: the chunk's K and V fragments
+      // are the same for every query block, and kept from one to the next
+      // they spilled
+      int z = 0;
+      asm volatile("" : "+v"(z));
+      const int q = qb * 16 + fr;
+      const int qc = q < L ? q : L - 1;
+      float qf[QN];
+      const float* qp = base + qc * ld;
+      if constexpr (HD >= 16) {
+#pragma unroll
+        for (int s = 0; s < HD / 16; ++s) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(qp + 16 * s + 4 * fg);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) qf[4 * s + e] = v[e];
+        }
+      } else {
+#pragma unroll
+        for (int e = 0; e < QN; ++e) qf[e] = qp[QN * fg + e];
+      }
+      f32x4 S[CKB];
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb) {
+        S[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const char* kr = Ks + z + (kb * 16 + fr) * STR;
+        if constexpr (HD >= 16) {
+#pragma unroll
+          for (int s = 0; s < HD / 16; ++s) {
+            const f32x4 kf = *reinterpret_cast<const f32x4*>(kr + (4 * s + fg) * 16);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[4 * s + e], S[kb], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < QN; ++e) {
+            const float kf = *reinterpret_cast<const float*>(kr + (QN * fg + e) * 4);
+            S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf, qf[e], S[kb], 0, 0, 0);
+          }
+        }
+        // here and below: keeps the scheduler from raising every LDS or mask
+        // read to the top, which spilled
+        if (kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      // lane: query fr, keys k0 + 16 kb + 4 fg + r.  With a mask tensor the
+      // logits are scaled and masked here, (logit - max) log2(e) is the
+      // exponent (a row of lowest-value masks keeps its differences); without,
+      // the raw products stay and one FMA by scale log2(e) finishes each.
+      if constexpr (MT) {
+        const float* mrow = a.mask + ((int64_t)(win % a.nW_mask) * L + qc) * (int64_t)L + k0 + 4 * fg;
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb) {
+          if (k0 + kb * 16 + 16 <= L) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[kb][r] = fmaf(S[kb][r], a.scale, mrow[kb * 16 + r]);
+          } else if (k0 + kb * 16 < L) {        // the window ends in this block
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (k0 + kb * 16 + 4 * fg + r < L) S[kb][r] = fmaf(S[kb][r], a.scale, mrow[kb * 16 + r]);
+          }
+        }
+      } else if (shifted) {
+        const unsigned qcls = qc % wa >= thr ? 1u : 0u;
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb) {
+          const unsigned bits = *reinterpret_cast<const unsigned*>(cls + z + kb * 16 + 4 * fg);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (((bits >> (8 * r)) & 1u) != qcls) S[kb][r] += a.smask;
+        }
+      }
+      if (k0 + ROWS > L) {
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (k0 + kb * 16 + 4 * fg + r >= L) S[kb][r] = -INFINITY;
+      }
+      float cm = S[0][0];
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cm = fmaxf(cm, S[kb][r]);
+      const float mn = fmaxf(mx[i], rows4_max(cm));
+      // from 0 while every logit so far is -inf (keys masked by -inf)
+      const float mo = mn == -INFINITY ? 0.f : mn;
+      const float zs = MT ? LOG2E : a.zscale;
+      if (k0 > 0) {
+        const float corr = __builtin_amdgcn_exp2f((mx[i] - mo) * zs);
+        l[i] *= corr;
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) O[i][db][r] *= corr;
+      }
+      mx[i] = mn;
+      const float off = -mo * zs;
+      float zl = 0.f;
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[kb][r] = __builtin_amdgcn_exp2f(MT ? (S[kb][r] - mo) * zs : fmaf(S[kb][r], zs, off));
+          zl += S[kb][r];
+        }
+      l[i] += zl;
+      asm volatile("" : "+v"(z) : "v"(zl));   // and the V reads stay behind the softmax
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const char* vr = Vs + z + (kb * 16 + 4 * fg + r) * STR;
+#pragma unroll
+          for (int db = 0; db < NDB; ++db) {
+            const float v = *reinterpret_cast<const float*>(vr + (16 * db + (HD >= 16 ? fr : fr % HD)) * 4);
+            O[i][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[i][db], 0, 0, 0);
+          }
+        }
+        if (HD != 64 || kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
-  NSW_WAIT_VMCNT(0);
-  wg_barrier();
-
-  const float* base = (const float*)a.qkv + (int64_t)win * L * ld + head * HD;
-  const char* Ks = smem;
-  const char* Vs = smem + PART;
-  const float zscale = a.scale * LOG2E;
-  const float smask = -100.0f / a.scale;
 #pragma unroll
   for (int i = 0; i < QPW; ++i) {
     const int qb = wave + NW * i;
-    if (qb >= NKB) break;
+    if (qb >= nqb) break;
     const int q = qb * 16 + fr;
-    const int qc = q < L ? q : L - 1;
-    f32x4 qf[NS];
+    const float inv = 1.0f / rows4_sum(l[i]);
+    float* orow = (float*)a.o + ((int64_t)win * L + q) * (int64_t)a.C + head * HD;
+    // lane (i, g): O[query i][16 db + 4g .. +3]
 #pragma unroll
-    for (int s = 0; s < NS; ++s) qf[s] = *reinterpret_cast<const f32x4*>(base + (int64_t)qc * ld + 16 * s + 4 * fg);
-    // S^T = K Q^T
-    f32x4 S[NKB];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb) {
-      S[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const int r = kb * 16 + fr;
-#pragma unroll
-      for (int s = 0; s < NS; ++s) {
-        const f32x4 kf = *reinterpret_cast<const f32x4*>(Ks + r * (HD * 4) + (((4 * s + fg) ^ (r & 15)) * 16));
-#pragma unroll
-        for (int e = 0; e < 4; ++e) S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[s][e], S[kb], 0, 0, 0);
-      }
-    }
-    // lane: query fr, keys 16 kb + 4 fg + r
-    if (shifted) {
-      const int qcls = (int)((cls[qc >> 6] >> (qc & 63)) & 1);
-#pragma unroll
-      for (int kb = 0; kb < NKB; ++kb) {
-        const unsigned bits = (unsigned)(cls[kb >> 2] >> (16 * (kb & 3) + 4 * fg)) & 0xFu;
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if ((int)((bits >> r) & 1u) != qcls) S[kb][r] += smask;
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if ((NKB - 1) * 16 + 4 * fg + r >= L) S[NKB - 1][r] = -INFINITY;
-    float mx = S[0][0];
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) mx = fmaxf(mx, S[kb][r]);
-    mx = rows4_max(mx);
-    const float off = -mx * zscale;
-    float zl = 0.f;
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        S[kb][r] = __builtin_amdgcn_exp2f(fmaf(S[kb][r], zscale, off));
-        zl += S[kb][r];
-      }
-    const float z = rows4_sum(zl);
-    // O^T = V^T P^T
-    f32x4 O[NDB];
-#pragma unroll
-    for (int db = 0; db < NDB; ++db) O[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int row = kb * 16 + 4 * fg + r;
-        const char* vr = Vs + row * (HD * 4) + (fr & 3) * 4;
-#pragma unroll
-        for (int db = 0; db < NDB; ++db) {
-          const float v = *reinterpret_cast<const float*>(vr + (((4 * db + fr / 4) ^ (fg << 2)) * 16));
-          O[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[db], 0, 0, 0);
-        }
-      }
-    if (q < L) {
-      const float inv = 1.0f / z;
-      float* orow = (float*)a.o + ((int64_t)win * L + q) * (int64_t)C + head * HD + 4 * fg;
-#pragma unroll
-      for (int db = 0; db < NDB; ++db)
-        *reinterpret_cast<f32x4*>(orow + 16 * db) =
-            f32x4{O[db][0] * inv, O[db][1] * inv, O[db][2] * inv, O[db][3] * inv};
-    }
+    for (int db = 0; db < NDB; ++db)
+      if (q < L && 16 * db + 4 * fg < HD)
+        *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * fg) =
+            f32x4{O[i][db][0] * inv, O[i][db][1] * inv, O[i][db][2] * inv, O[i][db][3] * inv};
   }
 }
 
-// ------------------------------------------------------- generic (fp32) ----
+// -------------------------------------------------------------- generic ----
 template <typename T, int HD>
 __global__ __launch_bounds__(256) void attn_scalar_kernel(AttnArgs a) {
   constexpr int KC = 64;  // keys per LDS chunk
@@ -885,15 +953,39 @@ static int launch_dma(const AttnArgs& a0, int64_t items, hipStream_t st) {
   return 0;
 }
 
-// fp32, head dim 64 without a mask tensor, 9 x 18 windows: attn_f32_kernel
-// (conditions as launch_dma, with 4-byte elements).
-static int launch_f32(const AttnArgs& a, int64_t items, hipStream_t st) {
-  const int nkb = (a.L + 15) / 16;
-  const uint64_t qkv_bytes = (uint64_t)items / a.heads * a.L * 3ull * a.C * 4ull;
-  if (nkb != 11 || qkv_bytes >= (1ull << 31) || items >= (1ll << 31) || items % a.heads != 0) return -1;
-  if ((uintptr_t)a.qkv % 16 != 0 || (uintptr_t)a.o % 16 != 0) return -1;
-  hipLaunchKernelGGL((attn_f32_kernel<11>), dim3((unsigned)items), dim3(512), 0, st, a, (int)items);
+// fp32 MFMA attention.  Returns -1 when it does not apply: windows above 384
+// tokens, unaligned tensors, a scale that is not positive (the row maximum is
+// taken of the raw products) or whose -100 / scale is not finite.
+template <int HD>
+static int launch_f32_mfma_hd(const AttnArgs& a, int64_t items, hipStream_t st) {
+  const bool mt = a.mask_mode == MASK_TENSOR;
+  if (a.L <= 192) {
+    if (mt) hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 4, true>), dim3((unsigned)items), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 4, false>), dim3((unsigned)items), dim3(256), 0, st, a);
+  } else {
+    if (mt) hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 8, true>), dim3((unsigned)items), dim3(512), 0, st, a);
+    else hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 8, false>), dim3((unsigned)items), dim3(512), 0, st, a);
+  }
   return 0;
+}
+
+static int launch_f32_mfma(const AttnArgs& a0, int hd, int64_t items, hipStream_t st) {
+  if (a0.L > 384 || items >= (1ll << 31)) return -1;
+  if ((uintptr_t)a0.qkv % 16 != 0 || (uintptr_t)a0.o % 16 != 0) return -1;
+  AttnArgs a = a0;
+  a.zscale = a.scale * 1.4426950408889634f;
+  a.smask = -100.0f / a.scale;
+  if (!(a.scale > 0.f) || !std::isfinite(a.zscale) || !std::isfinite(a.smask)) return -1;
+  a.dheads = FastDiv::make((uint32_t)a.heads);
+  switch (hd) {
+    case 4: return launch_f32_mfma_hd<4>(a, items, st);
+    case 8: return launch_f32_mfma_hd<8>(a, items, st);
+    case 16: return launch_f32_mfma_hd<16>(a, items, st);
+    case 32: return launch_f32_mfma_hd<32>(a, items, st);
+    case 64: return launch_f32_mfma_hd<64>(a, items, st);
+    case 128: return launch_f32_mfma_hd<128>(a, items, st);
+    default: return -1;
+  }
 }
 
 template <typename T>
@@ -955,7 +1047,7 @@ extern "C" int nsw_window_attention(const void* qkv, void* o, const float* mask,
     if (rc != 0) rc = launch_scalar<bf16>(a, hd, grid, st);
     if (rc != 0) return set_error(NSW_ERR_UNSUPPORTED, "%s: head_dim=%d, L=%lld unsupported", what, hd, (long long)L);
   } else if (dtype == NSW_DTYPE_F32) {
-    if (hd == 64 && a.mask_mode != MASK_TENSOR && launch_f32(a, grid, st) == 0) return check_launch(what);
+    if (launch_f32_mfma(a, hd, grid, st) == 0) return check_launch(what);
     if (launch_scalar<float>(a, hd, grid, st) != 0)
       return set_error(NSW_ERR_UNSUPPORTED, "%s: head_dim=%d unsupported (4, 8, 16, 32, 64, 128)", what, hd);
   } else {
