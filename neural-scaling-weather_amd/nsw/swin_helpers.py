@@ -21,7 +21,7 @@ import torch
 import torch.nn as nn
 
 from . import _lib, ops, torch_ops
-from .layer_helpers import BiasLayer, LinearLayer, NormLayer
+from .layer_helpers import BiasLayer, LinearLayer, NormLayer, parameter, submodule
 from .mlp import MLP
 from .profiler_utils import profile
 
@@ -111,10 +111,12 @@ class WindowMultiHeadAttention(nn.Module):
     def packed_qkv(self):
         """[Wq;Wk;Wv] and [bq;bk;bv], rebuilt when a parameter changes (not
         cached while torch.compile traces: the cache key reads data_ptr)."""
-        ps = (self.q.weight, self.k.weight, self.v.weight, self.biasq.bias, self.biask.bias, self.biasv.bias)
         if torch.compiler.is_compiling():
+            ps = (self.q.weight, self.k.weight, self.v.weight, self.biasq.bias, self.biask.bias, self.biasv.bias)
             return (torch.cat([p.detach() for p in ps[:3]], 0).contiguous(),
                     torch.cat([p.detach() for p in ps[3:]], 0).contiguous())
+        ps = ([parameter(submodule(self, n), "weight") for n in ("q", "k", "v")]
+              + [parameter(submodule(self, n), "bias") for n in ("biasq", "biask", "biasv")])
         key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps)
         if key != self._pack_key:
             with torch.no_grad():
@@ -201,7 +203,10 @@ class Block(nn.Module):
         return self.attn_mask.to(device=device, dtype=torch.float32)
 
     def _eps(self, dtype) -> float:
-        es = {_eps_of(n, dtype) for n in (self.norm1, self.norm2, self.attn.q_norm, self.attn.k_norm)}
+        sub = getattr if torch.compiler.is_compiling() else submodule
+        a = sub(self, "attn")
+        es = {sub(sub(o, n), "norm").eps for o, n in ((self, "norm1"), (self, "norm2"), (a, "q_norm"), (a, "k_norm"))}
+        es = {float(torch.finfo(dtype).eps) if e is None else float(e) for e in es}
         if len(es) != 1:
             raise NotImplementedError("the fused block needs one eps for all four RMSNorms")
         return es.pop()
@@ -210,16 +215,18 @@ class Block(nn.Module):
         """Tensors named like the fields of nsw_block_params.  The norm-folded
         weights are included as fold_norm1 / fold_norm2 ask, or both when
         ``fold_all`` (the window-order chain of SwinTransformer.forward)."""
-        a = self.attn
         fold1 = self.fold_norm1 or fold_all
         fold2 = self.fold_norm2 or fold1
         if torch.compiler.is_compiling():
             # traced: built from the parameters each call (the cache key reads data_ptr)
             return self._build_pack(fold1, fold2)
-        ps = [self.norm1.norm.weight, a.q.weight, a.k.weight, a.v.weight, a.biasq.bias, a.biask.bias,
-              a.biasv.bias, a.q_norm.norm.weight, a.k_norm.norm.weight, a.proj.weight, a.biasproj.bias,
-              self.norm2.norm.weight, self.mlp.fc1.weight, self.mlp.bias1.bias, self.mlp.fc2.weight,
-              self.mlp.bias2.bias]
+        a, m = submodule(self, "attn"), submodule(self, "mlp")
+        ps = [parameter(submodule(a, n), "weight") for n in ("q", "k", "v", "proj")]
+        ps += [parameter(submodule(a, n), "bias") for n in ("biasq", "biask", "biasv", "biasproj")]
+        ps += [parameter(submodule(m, n), "weight") for n in ("fc1", "fc2")]
+        ps += [parameter(submodule(m, n), "bias") for n in ("bias1", "bias2")]
+        ps += [parameter(submodule(submodule(o, n), "norm"), "weight")
+               for o, n in ((self, "norm1"), (self, "norm2"), (a, "q_norm"), (a, "k_norm"))]
         key = tuple((p.data_ptr(), p._version, p.dtype, p.device) for p in ps)
         if key != self._pack_key:
             self._pack = self._build_pack(False, False)
