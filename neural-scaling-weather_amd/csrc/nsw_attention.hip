@@ -634,9 +634,12 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 //     below 16) of key row i (A) and query i (B), so lane (i, g) holds the
 //     logits of query i for keys 16kb + 4g + r;
 //   O^T = V^T P^T: for key step (kb, r) lane (i, g) supplies V[16kb + 4g + r]
-//     [16db + i] (A) and its own probability (B); below head dim 16 the lanes
-//     past the head repeat its dims and are not stored (head dim 4 on the VALU
-//     instead spilled).
+//     [16db + i] (A) and its own probability (B).
+// Head dims 4 and 8 form O^T with v_mfma_f32_4x4x1_16b_f32 (8 cycles; a 16 x 16 x
+// 4 block takes 32 and would use 4 or 8 of its 16 rows): block (g, i / 4) takes
+// V[16kb + 4g + r][4db + i % 4] (A) and the lane's own probability (B), so lane
+// (i, g) sums query i over the keys of its group, and the four groups are added
+// at the end.  V is transposed in LDS there: one read gives a lane's four keys.
 // Rows are padded by 16 bytes in LDS: fragment reads (16 rows, one chunk) and the
 // V reads (4 rows 4 apart, 64 bytes each) then cover every bank once.
 // Probabilities, sums and outputs stay fp32.  Bound by the fp32 matrix rate and
@@ -644,12 +647,17 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 // tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
 // others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
 // 540; the same 200 x 8 with a mask tensor: 830 / 214; 100 x 6 of 32: 132 / 47;
-// 400 windows of 324, 8 heads of 4: 630 / 212; 100 x 8 of 64: 1226 / 293.
+// 400 windows of 324, 8 heads of 4: 630 / 174 (212
+// with the wide blocks); 100 x 8 of 64: 1226 / 293.
 template <int HD> struct AttnF32 {
   static constexpr int STR = HD == 4 ? 16 : HD * 4 + 16;       // bytes per K / V row
   static constexpr int CKB = HD <= 32 ? 11 : HD == 64 ? 6 : 3; // 16-key blocks per chunk
   static constexpr int ROWS = CKB * 16;
-  static constexpr int NDB = HD >= 16 ? HD / 16 : 1;           // 16-wide output blocks
+  static constexpr bool NARROW = HD < 16;
+  static constexpr int DB = NARROW ? 4 : 16;                   // head dims per output block
+  static constexpr int NDB = HD / DB;
+  static constexpr int VSTR = ROWS * 4;                        // NARROW: bytes per head dim of V^T
+  static constexpr int VBYTES = NARROW ? HD * VSTR : ROWS * STR;
   static constexpr int QN = HD / 4;                            // head dims per lane group
 };
 
@@ -660,7 +668,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
   constexpr int QPW = 3;
   constexpr float LOG2E = 1.4426950408889634f;
   __shared__ __attribute__((aligned(16))) char Ks[ROWS * STR];
-  __shared__ __attribute__((aligned(16))) char Vs[ROWS * STR];
+  __shared__ __attribute__((aligned(16))) char Vs[F::VBYTES];
   __shared__ __attribute__((aligned(4))) unsigned char cls[ROWS];   // shift-mask class of the chunk's keys
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -699,7 +707,12 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
         vv = *reinterpret_cast<const f32x4*>(p + 2 * a.C);
       }
       *reinterpret_cast<f32x4*>(Ks + row * STR + c * 16) = kv;
-      *reinterpret_cast<f32x4*>(Vs + row * STR + c * 16) = vv;
+      if constexpr (F::NARROW) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(Vs + (4 * c + e) * F::VSTR + row * 4) = vv[e];
+      } else {
+        *reinterpret_cast<f32x4*>(Vs + row * STR + c * 16) = vv;
+      }
     }
     if (shifted)
       for (int row = tid; row < ROWS; row += NW * 64) cls[row] = (k0 + row) % wa >= thr ? 1 : 0;
@@ -816,13 +829,24 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
       asm volatile("" : "+v"(z) : "v"(zl));   // and the V reads stay behind the softmax
 #pragma unroll
       for (int kb = 0; kb < CKB; ++kb) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const char* vr = Vs + z + (kb * 16 + 4 * fg + r) * STR;
+        if constexpr (F::NARROW) {
+          static_assert(F::VSTR / 4 % 64 == 48, "the four head dims of a read lie in other banks");
 #pragma unroll
           for (int db = 0; db < NDB; ++db) {
-            const float v = *reinterpret_cast<const float*>(vr + (16 * db + (HD >= 16 ? fr : fr % HD)) * 4);
-            O[i][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[i][db], 0, 0, 0);
+            const f32x4 v = *reinterpret_cast<const f32x4*>(Vs + z + (4 * db + (fr & 3)) * F::VSTR +
+                                                            (kb * 16 + 4 * fg) * 4);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) O[i][db] = __builtin_amdgcn_mfma_f32_4x4x1f32(v[r], S[kb][r], O[i][db], 0, 0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const char* vr = Vs + z + (kb * 16 + 4 * fg + r) * STR;
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) {
+              const float v = *reinterpret_cast<const float*>(vr + (16 * db + fr) * 4);
+              O[i][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[i][db], 0, 0, 0);
+            }
           }
         }
         if (HD != 64 || kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
@@ -836,12 +860,22 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
     const int q = qb * 16 + fr;
     const float inv = 1.0f / rows4_sum(l[i]);
     float* orow = (float*)a.o + ((int64_t)win * L + q) * (int64_t)a.C + head * HD;
-    // lane (i, g): O[query i][16 db + 4g .. +3]
+    if constexpr (F::NARROW) {
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
-      if (q < L && 16 * db + 4 * fg < HD)
-        *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * fg) =
-            f32x4{O[i][db][0] * inv, O[i][db][1] * inv, O[i][db][2] * inv, O[i][db][3] * inv};
+      for (int db = 0; db < NDB; ++db) {
+        f32x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = rows4_sum(O[i][db][r]) * inv;
+        if (q < L && fg == db) *reinterpret_cast<f32x4*>(orow + 4 * db) = o;
+      }
+    } else {
+      // lane (i, g): O[query i][16 db + 4g .. +3]
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        if (q < L)
+          *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * fg) =
+              f32x4{O[i][db][0] * inv, O[i][db][1] * inv, O[i][db][2] * inv, O[i][db][3] * inv};
+    }
   }
 }
 
