@@ -624,22 +624,17 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------- fp32 MFMA ----
-// fp32 for every head dim, windows of up to 384 tokens, shift mask from indices,
-// a mask tensor or none.  One workgroup of NW waves per (window, head); wave w
+// fp32, head dims 16 to 128 (4 and 8: attn_f32_narrow_kernel), windows of up to
+// 384 tokens, shift mask from indices, a mask tensor or none.  One workgroup of NW waves per (window, head); wave w
 // owns the query blocks w, w + NW, w + 2 NW.  K and V pass through LDS in chunks
 // of CKB 16-key blocks (at most 48 KB, so that three workgroups share a CU);
 // each query block keeps its output, row maximum and row sum in registers from
 // chunk to chunk (online softmax).  v_mfma_f32_16x16x4_f32:
-//   S^T = K Q^T: lane group g supplies head dims 16s + 4g + e (hd / 4 per group
-//     below 16) of key row i (A) and query i (B), so lane (i, g) holds the
-//     logits of query i for keys 16kb + 4g + r;
+//   S^T = K Q^T: lane group g supplies head dims 16s + 4g + e of key row i (A)
+//     and query i (B), so lane (i, g) holds the logits of query i for keys
+//     16kb + 4g + r;
 //   O^T = V^T P^T: for key step (kb, r) lane (i, g) supplies V[16kb + 4g + r]
 //     [16db + i] (A) and its own probability (B).
-// Head dims 4 and 8 form O^T with v_mfma_f32_4x4x1_16b_f32 (8 cycles; a 16 x 16 x
-// 4 block takes 32 and would use 4 or 8 of its 16 rows): block (g, i / 4) takes
-// V[16kb + 4g + r][4db + i % 4] (A) and the lane's own probability (B), so lane
-// (i, g) sums query i over the keys of its group, and the four groups are added
-// at the end.  V is transposed in LDS there: one read gives a lane's four keys.
 // Rows are padded by 16 bytes in LDS: fragment reads (16 rows, one chunk) and the
 // V reads (4 rows 4 apart, 64 bytes each) then cover every bank once.
 // Probabilities, sums and outputs stay fp32.  Bound by the fp32 matrix rate and
@@ -647,17 +642,12 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 // tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
 // others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
 // 540; the same 200 x 8 with a mask tensor: 830 / 214; 100 x 6 of 32: 132 / 47;
-// 400 windows of 324, 8 heads of 4: 630 / 174 (212
-// with the wide blocks); 100 x 8 of 64: 1226 / 293.
+// 100 x 8 of 64: 1226 / 293.
 template <int HD> struct AttnF32 {
-  static constexpr int STR = HD == 4 ? 16 : HD * 4 + 16;       // bytes per K / V row
+  static constexpr int STR = HD * 4 + 16;                      // bytes per K / V row
   static constexpr int CKB = HD <= 32 ? 11 : HD == 64 ? 6 : 3; // 16-key blocks per chunk
   static constexpr int ROWS = CKB * 16;
-  static constexpr bool NARROW = HD < 16;
-  static constexpr int DB = NARROW ? 4 : 16;                   // head dims per output block
-  static constexpr int NDB = HD / DB;
-  static constexpr int VSTR = ROWS * 4;                        // NARROW: bytes per head dim of V^T
-  static constexpr int VBYTES = NARROW ? HD * VSTR : ROWS * STR;
+  static constexpr int NDB = HD / 16;                          // 16-wide output blocks
   static constexpr int QN = HD / 4;                            // head dims per lane group
 };
 
@@ -668,7 +658,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
   constexpr int QPW = 3;
   constexpr float LOG2E = 1.4426950408889634f;
   __shared__ __attribute__((aligned(16))) char Ks[ROWS * STR];
-  __shared__ __attribute__((aligned(16))) char Vs[F::VBYTES];
+  __shared__ __attribute__((aligned(16))) char Vs[ROWS * STR];
   __shared__ __attribute__((aligned(4))) unsigned char cls[ROWS];   // shift-mask class of the chunk's keys
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -707,12 +697,7 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
         vv = *reinterpret_cast<const f32x4*>(p + 2 * a.C);
       }
       *reinterpret_cast<f32x4*>(Ks + row * STR + c * 16) = kv;
-      if constexpr (F::NARROW) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) *reinterpret_cast<float*>(Vs + (4 * c + e) * F::VSTR + row * 4) = vv[e];
-      } else {
-        *reinterpret_cast<f32x4*>(Vs + row * STR + c * 16) = vv;
-      }
+      *reinterpret_cast<f32x4*>(Vs + row * STR + c * 16) = vv;
     }
     if (shifted)
       for (int row = tid; row < ROWS; row += NW * 64) cls[row] = (k0 + row) % wa >= thr ? 1 : 0;
@@ -730,35 +715,22 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
       const int qc = q < L ? q : L - 1;
       float qf[QN];
       const float* qp = base + qc * ld;
-      if constexpr (HD >= 16) {
 #pragma unroll
-        for (int s = 0; s < HD / 16; ++s) {
-          const f32x4 v = *reinterpret_cast<const f32x4*>(qp + 16 * s + 4 * fg);
+      for (int s = 0; s < HD / 16; ++s) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(qp + 16 * s + 4 * fg);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) qf[4 * s + e] = v[e];
-        }
-      } else {
-#pragma unroll
-        for (int e = 0; e < QN; ++e) qf[e] = qp[QN * fg + e];
+        for (int e = 0; e < 4; ++e) qf[4 * s + e] = v[e];
       }
       f32x4 S[CKB];
 #pragma unroll
       for (int kb = 0; kb < CKB; ++kb) {
         S[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
         const char* kr = Ks + z + (kb * 16 + fr) * STR;
-        if constexpr (HD >= 16) {
 #pragma unroll
-          for (int s = 0; s < HD / 16; ++s) {
-            const f32x4 kf = *reinterpret_cast<const f32x4*>(kr + (4 * s + fg) * 16);
+        for (int s = 0; s < HD / 16; ++s) {
+          const f32x4 kf = *reinterpret_cast<const f32x4*>(kr + (4 * s + fg) * 16);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[4 * s + e], S[kb], 0, 0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int e = 0; e < QN; ++e) {
-            const float kf = *reinterpret_cast<const float*>(kr + (QN * fg + e) * 4);
-            S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf, qf[e], S[kb], 0, 0, 0);
-          }
+          for (int e = 0; e < 4; ++e) S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[e], qf[4 * s + e], S[kb], 0, 0, 0);
         }
         // here and below: keeps the scheduler from raising every LDS or mask
         // read to the top, which spilled
@@ -829,24 +801,13 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
       asm volatile("" : "+v"(z) : "v"(zl));   // and the V reads stay behind the softmax
 #pragma unroll
       for (int kb = 0; kb < CKB; ++kb) {
-        if constexpr (F::NARROW) {
-          static_assert(F::VSTR / 4 % 64 == 48, "the four head dims of a read lie in other banks");
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const char* vr = Vs + z + (kb * 16 + 4 * fg + r) * STR;
 #pragma unroll
           for (int db = 0; db < NDB; ++db) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(Vs + z + (4 * db + (fr & 3)) * F::VSTR +
-                                                            (kb * 16 + 4 * fg) * 4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) O[i][db] = __builtin_amdgcn_mfma_f32_4x4x1f32(v[r], S[kb][r], O[i][db], 0, 0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const char* vr = Vs + z + (kb * 16 + 4 * fg + r) * STR;
-#pragma unroll
-            for (int db = 0; db < NDB; ++db) {
-              const float v = *reinterpret_cast<const float*>(vr + (16 * db + fr) * 4);
-              O[i][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[i][db], 0, 0, 0);
-            }
+            const float v = *reinterpret_cast<const float*>(vr + (16 * db + fr) * 4);
+            O[i][db] = __builtin_amdgcn_mfma_f32_16x16x4f32(v, S[kb][r], O[i][db], 0, 0, 0);
           }
         }
         if (HD != 64 || kb % 2 == 1) __builtin_amdgcn_sched_barrier(0);
@@ -860,21 +821,166 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
     const int q = qb * 16 + fr;
     const float inv = 1.0f / rows4_sum(l[i]);
     float* orow = (float*)a.o + ((int64_t)win * L + q) * (int64_t)a.C + head * HD;
-    if constexpr (F::NARROW) {
+    // lane (i, g): O[query i][16 db + 4g .. +3]
 #pragma unroll
-      for (int db = 0; db < NDB; ++db) {
-        f32x4 o;
+    for (int db = 0; db < NDB; ++db)
+      if (q < L)
+        *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * fg) =
+            f32x4{O[i][db][0] * inv, O[i][db][1] * inv, O[i][db][2] * inv, O[i][db][3] * inv};
+  }
+}
+
+// Head dims 4 and 8: the whole window's K and V (at most 32 KB) lie in LDS,
+// transposed, so that a wave takes its query blocks one after the other (wave,
+// wave + 4, ...) with one block's output in registers, and nothing is waited for
+// after the first barrier.  Up to 176 tokens are one chunk of 11 blocks of 16
+// keys (162: 48.6 us in two chunks of 7); more pass in chunks of 7 (324: 3 whole
+// chunks) with an online softmax.
+//   S^T = K Q^T with v_mfma_f32_16x16x4_f32: instruction e takes head dim 4e + g
+//     from lane group g, so lane (i, g) holds query i's logits for keys 16kb +
+//     4g + r;
+//   O^T = V^T P^T with v_mfma_f32_4x4x1_16b_f32 (8 cycles; a 16 x 16 x 4 block
+//     takes 32 and would use 4 or 8 of its 16 rows): block (g, i / 4) takes
+//     V[16kb + 4g + r][4db + i % 4] (A) and the lane's own probability (B), so
+//     lane (i, g) sums query i over the keys of its group, and the four groups
+//     are added at the end.
+// KSTR: the four head dims of a K or V read lie in other banks (48 mod 64).
+// Bound by the softmax's VALU work.  400 windows of 324, 8 heads of 4: 630 us in
+// attn_scalar_kernel, 148 in the kernel above with 4 x 4 x 1 blocks, 123 here (of
+// 162 tokens: 43 / 39); 8 heads of 8: 197 / 185.
+template <int HD, bool MT, int CKB>
+__global__ __launch_bounds__(256, 5) void attn_f32_narrow_kernel(AttnArgs a) {
+  constexpr int ROWS = CKB * 16, NDB = HD / 4;
+  constexpr int MAXR = CKB == 11 ? ROWS : (384 + ROWS - 1) / ROWS * ROWS;   // 11: one chunk
+  constexpr int KSTR = MAXR + (48 - MAXR % 64 + 64) % 64;
+  static_assert(KSTR % 64 == 48 && KSTR % 4 == 0, "LDS layout");
+  constexpr float LOG2E = 1.4426950408889634f;
+  __shared__ __attribute__((aligned(16))) float Kt[HD * KSTR];
+  __shared__ __attribute__((aligned(16))) float Vt[HD * KSTR];
+  __shared__ __attribute__((aligned(4))) unsigned char cls[MAXR];   // shift-mask class of the keys
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int fr = lane & 15, fg = lane >> 4;
+  const int L = a.L;
+  const int64_t ld = 3 * (int64_t)a.C;
+  const uint32_t item = (uint32_t)xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const uint32_t win = a.dheads.div(item);
+  const int head = (int)(item - win * (uint32_t)a.heads);
+  const float* base = (const float*)a.qkv + (int64_t)win * L * ld + head * HD;
+  const bool shifted = !MT && window_in_last_band(a, win);
+  const int thr = shifted ? (a.g.ws0 - a.g.s0) * a.g.ws1 : 0, wa = shifted ? a.g.wa : 1;
+  const int nqb = (L + 15) / 16;
+
+  for (int row = tid; row < (L + ROWS - 1) / ROWS * ROWS; row += 256) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) o[r] = rows4_sum(O[i][db][r]) * inv;
-        if (q < L && fg == db) *reinterpret_cast<f32x4*>(orow + 4 * db) = o;
+    for (int c = 0; c < NDB; ++c) {
+      f32x4 kv = {0.f, 0.f, 0.f, 0.f}, vv = kv;
+      if (row < L) {
+        const float* p = base + row * ld + 4 * c;
+        kv = *reinterpret_cast<const f32x4*>(p + a.C);
+        vv = *reinterpret_cast<const f32x4*>(p + 2 * a.C);
       }
-    } else {
-      // lane (i, g): O[query i][16 db + 4g .. +3]
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        Kt[(4 * c + e) * KSTR + row] = kv[e];
+        Vt[(4 * c + e) * KSTR + row] = vv[e];
+      }
+    }
+    if (shifted) cls[row] = row % wa >= thr ? 1 : 0;
+  }
+  __syncthreads();
+
+  for (int qb = wave; qb < nqb; qb += 4) {
+    const int q = qb * 16 + fr;
+    const int qc = q < L ? q : L - 1;
+    float qf[NDB];
+#pragma unroll
+    for (int e = 0; e < NDB; ++e) qf[e] = base[qc * ld + 4 * e + fg];
+    f32x4 O[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) O[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float mx = -INFINITY, l = 0.f;
+    for (int k0 = 0; k0 < L; k0 += ROWS) {
+      f32x4 S[CKB];
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb) {
+        S[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < NDB; ++e)
+          S[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(Kt[(4 * e + fg) * KSTR + k0 + kb * 16 + fr], qf[e], S[kb], 0, 0, 0);
+      }
+      if constexpr (MT) {
+        const float* mrow = a.mask + ((int64_t)(win % a.nW_mask) * L + qc) * (int64_t)L + k0 + 4 * fg;
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb) {
+          if (k0 + kb * 16 + 16 <= L) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[kb][r] = fmaf(S[kb][r], a.scale, mrow[kb * 16 + r]);
+          } else if (k0 + kb * 16 < L) {        // the window ends in this block
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (k0 + kb * 16 + 4 * fg + r < L) S[kb][r] = fmaf(S[kb][r], a.scale, mrow[kb * 16 + r]);
+          }
+        }
+      } else if (shifted) {
+        const unsigned qcls = qc % wa >= thr ? 1u : 0u;
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb) {
+          const unsigned bits = *reinterpret_cast<const unsigned*>(cls + k0 + kb * 16 + 4 * fg);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (((bits >> (8 * r)) & 1u) != qcls) S[kb][r] += a.smask;
+        }
+      }
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+        if (k0 + kb * 16 + 16 > L) {            // past the window in this block
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (k0 + kb * 16 + 4 * fg + r >= L) S[kb][r] = -INFINITY;
+        }
+      float cm = S[0][0];
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) cm = fmaxf(cm, S[kb][r]);
+      const float mn = fmaxf(mx, rows4_max(cm));
+      // from 0 while every logit so far is -inf (keys masked by -inf)
+      const float mo = mn == -INFINITY ? 0.f : mn;
+      const float zs = MT ? LOG2E : a.zscale;
+      const float corr = __builtin_amdgcn_exp2f((mx - mo) * zs);   // 0 in the first chunk
+      l *= corr;
 #pragma unroll
       for (int db = 0; db < NDB; ++db)
-        if (q < L)
-          *reinterpret_cast<f32x4*>(orow + 16 * db + 4 * fg) =
-              f32x4{O[i][db][0] * inv, O[i][db][1] * inv, O[i][db][2] * inv, O[i][db][3] * inv};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) O[db][r] *= corr;
+      mx = mn;
+      const float off = -mo * zs;
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          S[kb][r] = __builtin_amdgcn_exp2f(MT ? (S[kb][r] - mo) * zs : fmaf(S[kb][r], zs, off));
+          l += S[kb][r];
+        }
+#pragma unroll
+      for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          const f32x4 v = *reinterpret_cast<const f32x4*>(Vt + (4 * db + (fr & 3)) * KSTR + k0 + kb * 16 + 4 * fg);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) O[db] = __builtin_amdgcn_mfma_f32_4x4x1f32(v[r], S[kb][r], O[db], 0, 0, 0);
+        }
+    }
+    const float inv = 1.0f / rows4_sum(l);
+    float* orow = (float*)a.o + ((int64_t)win * L + q) * (int64_t)a.C + head * HD;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) {
+      f32x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = rows4_sum(O[db][r]) * inv;
+      if (q < L && fg == db) *reinterpret_cast<f32x4*>(orow + 4 * db) = o;
     }
   }
 }
@@ -1003,6 +1109,19 @@ static int launch_f32_mfma_hd(const AttnArgs& a, int64_t items, hipStream_t st) 
   return 0;
 }
 
+template <int HD>
+static int launch_f32_narrow(const AttnArgs& a, int64_t items, hipStream_t st) {
+  const bool mt = a.mask_mode == MASK_TENSOR;
+  if (a.L <= 176) {
+    if (mt) hipLaunchKernelGGL((attn_f32_narrow_kernel<HD, true, 11>), dim3((unsigned)items), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((attn_f32_narrow_kernel<HD, false, 11>), dim3((unsigned)items), dim3(256), 0, st, a);
+  } else {
+    if (mt) hipLaunchKernelGGL((attn_f32_narrow_kernel<HD, true, 7>), dim3((unsigned)items), dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((attn_f32_narrow_kernel<HD, false, 7>), dim3((unsigned)items), dim3(256), 0, st, a);
+  }
+  return 0;
+}
+
 static int launch_f32_mfma(const AttnArgs& a0, int hd, int64_t items, hipStream_t st) {
   if (a0.L > 384 || items >= (1ll << 31)) return -1;
   if ((uintptr_t)a0.qkv % 16 != 0 || (uintptr_t)a0.o % 16 != 0) return -1;
@@ -1012,8 +1131,8 @@ static int launch_f32_mfma(const AttnArgs& a0, int hd, int64_t items, hipStream_
   if (!(a.scale > 0.f) || !std::isfinite(a.zscale) || !std::isfinite(a.smask)) return -1;
   a.dheads = FastDiv::make((uint32_t)a.heads);
   switch (hd) {
-    case 4: return launch_f32_mfma_hd<4>(a, items, st);
-    case 8: return launch_f32_mfma_hd<8>(a, items, st);
+    case 4: return launch_f32_narrow<4>(a, items, st);
+    case 8: return launch_f32_narrow<8>(a, items, st);
     case 16: return launch_f32_mfma_hd<16>(a, items, st);
     case 32: return launch_f32_mfma_hd<32>(a, items, st);
     case 64: return launch_f32_mfma_hd<64>(a, items, st);

@@ -73,3 +73,34 @@ def test_attention_f32_scales(scale):
     mask = torch.zeros(4, 162, 162, device="cuda:0")
     mask[2:] = torch.where(r[:, None] != r[None], -100.0, 0.0)
     assert _rel(o, _ref(qkv, 2, scale, mask)) < 1e-5
+
+
+# head dims 4 and 8 pass keys in chunks of 7 blocks (112): around one, two and three
+# chunks, with the shift mask from indices, a mask tensor (a whole leading chunk of
+# -inf in one row) and none; the bound as above
+@pytest.mark.parametrize("hd,heads", [(4, 3), (8, 2)])
+@pytest.mark.parametrize("L", [15, 16, 111, 112, 113, 224, 225, 336, 337])
+@pytest.mark.parametrize("kind", ["none", "mask"])
+def test_attention_f32_narrow_chunks(hd, heads, L, kind):
+    C = 16 * ((hd * heads + 15) // 16)
+    heads = C // hd
+    qkv = _qkv(3, L, C, L + hd)
+    mask = None
+    if kind == "mask":
+        g = torch.Generator(device="cuda:0").manual_seed(L)
+        mask = torch.randn(3, L, L, generator=g, device="cuda:0")
+        mask[1, 0, : L - 1] = float("-inf")
+    o = nsw.ops.window_attention(qkv, heads, hd ** -0.5, mask=mask)
+    assert _rel(o, _ref(qkv, heads, hd ** -0.5, mask)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
+
+
+@pytest.mark.parametrize("hd", [4, 8])
+@pytest.mark.parametrize("T", [1, 2])
+def test_attention_f32_narrow_shift(hd, T):
+    H, W, L = 18, 36, 162 * T
+    qkv = _qkv(4, L, 32, T)
+    o = nsw.ops.window_attention(qkv, 32 // hd, hd ** -0.5, geometry=(H, W, (9, 18), (4, 9), T))
+    r = torch.arange(L, device="cuda:0") % 162 // 18 >= 5
+    mask = torch.zeros(4, L, L, device="cuda:0")
+    mask[2:] = torch.where(r[:, None] != r[None], -100.0, 0.0)
+    assert _rel(o, _ref(qkv, 32 // hd, hd ** -0.5, mask)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
