@@ -641,8 +641,33 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 // the softmax's VALU work.  Measured, us, before (head dim 64, 9 x 18, no mask
 // tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
 // others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
-// 540; the same 200 x 8 with a mask tensor: 830 / 214; 100 x 6 of 32: 132 / 47;
+// 540; 200 x 8 with a mask tensor: 830 / 165
+// (213 with its values loaded after the products; 152 without one); 100 x 6 of 32: 132 / 47;
 // 100 x 8 of 64: 1226 / 293.
+// The mask values of a query for one chunk, keys 16 kb + 4 fg + r of n left in the
+// window (0 past them).  Rows of any L are 4-byte aligned
+// only, which 16-byte global loads allow.
+typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+template <int CKB>
+__device__ __forceinline__ void load_mask(f32x4 (&mk)[CKB], const float* mwin, int at, int n, int fg) {
+  if (n >= 16 * CKB) {
+#pragma unroll
+    for (int kb = 0; kb < CKB; ++kb) mk[kb] = *reinterpret_cast<const f32x4_a4*>(mwin + at + kb * 16);
+    return;
+  }
+#pragma unroll
+  for (int kb = 0; kb < CKB; ++kb) {
+    mk[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (kb * 16 + 16 <= n) {
+      mk[kb] = *reinterpret_cast<const f32x4_a4*>(mwin + at + kb * 16);
+    } else if (kb * 16 < n) {                   // the window ends in this block
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (kb * 16 + 4 * fg + r < n) mk[kb][r] = mwin[at + kb * 16 + r];
+    }
+  }
+}
+
 template <int HD> struct AttnF32 {
   static constexpr int STR = HD * 4 + 16;                      // bytes per K / V row
   static constexpr int CKB = HD <= 32 ? 11 : HD == 64 ? 6 : 3; // 16-key blocks per chunk
@@ -670,6 +695,11 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
   const uint32_t win = a.dheads.div(item);
   const int head = (int)(item - win * (uint32_t)a.heads);
   const float* base = (const float*)a.qkv + (int64_t)win * L * ld + head * HD;
+  // a mask tensor's values are loaded ahead of the products at head dim 64; at the
+  // others they spilled there (24 to 66 registers)
+  constexpr bool EARLY = MT && HD == 64;
+  const float* mwin =
+      EARLY ? a.mask + (int64_t)__builtin_amdgcn_readfirstlane((int)(win % a.nW_mask)) * L * L : nullptr;
   const bool shifted = !MT && window_in_last_band(a, win);
   const int thr = shifted ? (a.g.ws0 - a.g.s0) * a.g.ws1 : 0, wa = shifted ? a.g.wa : 1;
   const int nqb = (L + 15) / 16;
@@ -721,6 +751,8 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
 #pragma unroll
         for (int e = 0; e < 4; ++e) qf[4 * s + e] = v[e];
       }
+      f32x4 mk[EARLY ? CKB : 1];
+      if constexpr (EARLY) load_mask<CKB>(mk, mwin, qc * L + k0 + 4 * fg + z, L - k0, fg);
       f32x4 S[CKB];
 #pragma unroll
       for (int kb = 0; kb < CKB; ++kb) {
@@ -740,7 +772,12 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
       // logits are scaled and masked here, (logit - max) log2(e) is the
       // exponent (a row of lowest-value masks keeps its differences); without,
       // the raw products stay and one FMA by scale log2(e) finishes each.
-      if constexpr (MT) {
+      if constexpr (EARLY) {
+#pragma unroll
+        for (int kb = 0; kb < CKB; ++kb)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S[kb][r] = fmaf(S[kb][r], a.scale, mk[kb][r]);
+      } else if constexpr (MT) {
         const float* mrow = a.mask + ((int64_t)(win % a.nW_mask) * L + qc) * (int64_t)L + k0 + 4 * fg;
 #pragma unroll
         for (int kb = 0; kb < CKB; ++kb) {
