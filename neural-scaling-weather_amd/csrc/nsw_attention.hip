@@ -26,8 +26,8 @@
 // Workgroup ids are remapped so that the heads of a window share one XCD.
 // Padding keys get -inf logits; no FLOPs are counted for them.
 //
-// fp32 (attn_f32_mfma_kernel): any head dim and mask, windows of up to 384
-// tokens, on the fp32 matrix instructions.
+// fp32 (attn_f32_mfma_kernel; head dims 4 and 8: attn_f32_narrow_kernel): any
+// mask, windows of up to 384 tokens, on the fp32 matrix instructions.
 //
 // Generic path (attn_scalar_kernel: larger windows, bf16 at other head dims):
 // one thread per query, online softmax over 64-key chunks staged in LDS, fp32
@@ -624,29 +624,9 @@ __global__ __launch_bounds__(256, 3) void attn_dma_kernel(AttnArgs a) {
 }
 
 // ---------------------------------------------------------- fp32 MFMA ----
-// fp32, head dims 16 to 128 (4 and 8: attn_f32_narrow_kernel), windows of up to
-// 384 tokens, shift mask from indices, a mask tensor or none.  One workgroup of NW waves per (window, head); wave w
-// owns the query blocks w, w + NW, w + 2 NW.  K and V pass through LDS in chunks
-// of CKB 16-key blocks (at most 48 KB, so that three workgroups share a CU);
-// each query block keeps its output, row maximum and row sum in registers from
-// chunk to chunk (online softmax).  v_mfma_f32_16x16x4_f32:
-//   S^T = K Q^T: lane group g supplies head dims 16s + 4g + e of key row i (A)
-//     and query i (B), so lane (i, g) holds the logits of query i for keys
-//     16kb + 4g + r;
-//   O^T = V^T P^T: for key step (kb, r) lane (i, g) supplies V[16kb + 4g + r]
-//     [16db + i] (A) and its own probability (B).
-// Rows are padded by 16 bytes in LDS: fragment reads (16 rows, one chunk) and the
-// V reads (4 rows 4 apart, 64 bytes each) then cover every bank once.
-// Probabilities, sums and outputs stay fp32.  Bound by the fp32 matrix rate and
-// the softmax's VALU work.  Measured, us, before (head dim 64, 9 x 18, no mask
-// tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
-// others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
-// 540; 200 x 8 with a mask tensor: 830 / 165
-// (213 with its values loaded after the products; 152 without one); 100 x 6 of 32: 132 / 47;
-// 100 x 8 of 64: 1226 / 293.
 // The mask values of a query for one chunk, keys 16 kb + 4 fg + r of n left in the
-// window (0 past them).  Rows of any L are 4-byte aligned
-// only, which 16-byte global loads allow.
+// window (0 past them).  Rows of any L are 4-byte aligned only, which 16-byte
+// global loads allow.
 typedef float f32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int CKB>
 __device__ __forceinline__ void load_mask(f32x4 (&mk)[CKB], const float* mwin, int at, int n, int fg) {
@@ -668,6 +648,27 @@ __device__ __forceinline__ void load_mask(f32x4 (&mk)[CKB], const float* mwin, i
   }
 }
 
+// fp32, head dims 16 to 128 (4 and 8: attn_f32_narrow_kernel), windows of up to
+// 384 tokens, shift mask from indices, a mask tensor or none.  One workgroup of NW
+// waves per (window, head); wave w owns the query blocks w, w + NW, w + 2 NW.  K
+// and V pass through LDS in chunks of CKB 16-key blocks (at most 48 KB, so that
+// three workgroups share a CU); each query block keeps its output, row maximum and
+// row sum in registers from chunk to chunk (online softmax).
+// v_mfma_f32_16x16x4_f32:
+//   S^T = K Q^T: lane group g supplies head dims 16s + 4g + e of key row i (A)
+//     and query i (B), so lane (i, g) holds the logits of query i for keys
+//     16kb + 4g + r;
+//   O^T = V^T P^T: for key step (kb, r) lane (i, g) supplies V[16kb + 4g + r]
+//     [16db + i] (A) and its own probability (B).
+// Rows are padded by 16 bytes in LDS: fragment reads (16 rows, one chunk) and the
+// V reads (4 rows 4 apart, 64 bytes each) then cover every bank once.
+// Probabilities, sums and outputs stay fp32.  Bound by the fp32 matrix rate and
+// the softmax's VALU work.  Measured, us, before (head dim 64, 9 x 18, no mask
+// tensor: this scheme with all of K and V in LDS, one workgroup per CU; the
+// others: attn_scalar_kernel) / now: 400 windows of 162, 16 heads of 64: 575 /
+// 540; 200 x 8 with a mask tensor: 830 / 165 (213 with its values loaded after the
+// products; 152 without one); 100 x 6 of 32: 132 / 47;
+// 100 x 8 of 64: 1226 / 293.
 template <int HD> struct AttnF32 {
   static constexpr int STR = HD * 4 + 16;                      // bytes per K / V row
   static constexpr int CKB = HD <= 32 ? 11 : HD == 64 ? 6 : 3; // 16-key blocks per chunk
