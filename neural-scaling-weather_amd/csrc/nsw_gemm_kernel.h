@@ -701,6 +701,7 @@ __device__ __forceinline__ void mainloop_split3(char* smem, const float* __restr
     xs = xn;
   }
   NSW_WAIT_VMCNT(0);   // the copies past the last stage
+  wg_barrier();        // the ring is no longer read
 }
 
 // Whether one of the wave's results is not finite (the same on every lane).
@@ -719,29 +720,53 @@ __device__ __forceinline__ bool any_nonfinite(const f32x4 (&acc)[TC::NB][TC::MB]
 // fp32 results that are not finite are formed again with the fp32 matrix
 // instruction: an infinite operand (or one that bf16 rounds to infinity, above
 // 3.39e38) has no finite parts, so the split gives NaN where fp32 gives an
-// infinity or a finite sum.  Whole waves take the branch (operands straight
-// from global memory, one 16 x 16 block at a time); on finite data none does.
+// infinity or a finite sum.  Only these results are replaced.  Operands straight
+// from global memory; of a wave's 16 x 16 blocks those with such a result, a few at
+// a time through LDS (buf, a KB each; with a loop for every block in the code, the
+// loads could not run ahead).  On finite data no wave does.
 template <class TC>
-__device__ __forceinline__ void redo_nonfinite(const float* __restrict__ X, const float* __restrict__ Wt, int M, int N,
-                                               int K, int mw0, int nw0, f32x4 (&acc)[TC::NB][TC::MB], int lane) {
+__device__ __forceinline__ void redo_nonfinite(char* buf, const float* __restrict__ X, const float* __restrict__ Wt, int M,
+                                               int N, int K, int mw0, int nw0, f32x4 (&acc)[TC::NB][TC::MB], int wave,
+                                               int lane) {
+  constexpr int NB = TC::NB, MB = TC::MB, G = 4;
+  static_assert(TC::NW * G * 1024 <= Stg<float, TC>::SMEM, "LDS layout");
   if (!any_nonfinite<TC>(acc)) return;
   const int frow = lane & 15, fg = lane >> 4;
+  f32x4* c = reinterpret_cast<f32x4*>(buf) + wave * G * 64 + lane;
+  uint32_t left = 0;     // blocks to be formed again: bits nb MB + mb
 #pragma unroll
-  for (int nb = 0; nb < TC::NB; ++nb) {
-    const int n = nw0 + nb * 16 + frow;
-    const float* wp = Wt + (int64_t)(n < N ? n : N - 1) * K + 4 * fg;
-#pragma unroll
-    for (int mb = 0; mb < TC::MB; ++mb) {
-      const int m = mw0 + mb * 16 + frow;
+  for (int b = 0; b < NB * MB; ++b) {
+    const f32x4 v = acc[b / MB][b % MB] * 0.f;        // NaN where a value is not finite
+    if (__ballot(!((v[0] + v[1]) + (v[2] + v[3]) == 0.f)) != 0) left |= 1u << b;
+  }
+#pragma unroll 1
+  while (left != 0) {
+    uint32_t now = left;
+#pragma unroll 1
+    for (int g = 0; g < G && left != 0; ++g) {
+      const int b = __builtin_ctz(left);
+      left &= left - 1;
+      const int n = nw0 + b / MB * 16 + frow, m = mw0 + b % MB * 16 + frow;
+      const float* wp = Wt + (int64_t)(n < N ? n : N - 1) * K + 4 * fg;
       const float* xp = X + (int64_t)(m < M ? m : M - 1) * K + 4 * fg;
-      f32x4 c = {0.f, 0.f, 0.f, 0.f};
+      f32x4 a = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 8
       for (int k = 0; k < K; k += 16) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(wp + k);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(xp + k);
+        const f32x4 w = *reinterpret_cast<const f32x4*>(wp + k);
+        const f32x4 x = *reinterpret_cast<const f32x4*>(xp + k);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+        for (int e = 0; e < 4; ++e) a = __builtin_amdgcn_mfma_f32_16x16x4f32(w[e], x[e], a, 0, 0, 0);
       }
-      acc[nb][mb] = c;
+      c[g * 64] = a;
+    }
+    now ^= left;
+#pragma unroll
+    for (int b = 0; b < NB * MB; ++b) {
+      if (((now >> b) & 1) == 0) continue;
+      const f32x4 a = c[__builtin_popcount(now & ((1u << b) - 1)) * 64];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (!(acc[b / MB][b % MB][r] * 0.f == 0.f)) acc[b / MB][b % MB][r] = a[r];
     }
   }
 }
@@ -874,7 +899,7 @@ __global__ __launch_bounds__(TC::NW * 64, TC::MINW) void gemm_kernel(const T* __
 #pragma unroll
           for (int j = 0; j < MB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         mainloop_split3<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
-        redo_nonfinite<TC>(X, Wt, M, N, K, m0 + wm * WTM, n0 + wn * WTN, acc, lane0);
+        redo_nonfinite<TC>(smem, X, Wt, M, N, K, m0 + wm * WTM, n0 + wn * WTN, acc, wave, lane0);
       }
     }
   }

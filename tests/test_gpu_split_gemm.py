@@ -140,3 +140,20 @@ def test_tile_sizes(dtype, H, W, C):
         img = nsw.ops.head_unpatchify(x, wh, 1, ch, H * p, W * p, p)
         want = (d(x) @ d(wh).t()).view(H, W, ch, p, p).permute(2, 0, 3, 1, 4).reshape(1, 1, ch, H * p, W * p)
         close(img, want)
+
+
+@pytest.mark.parametrize("K", [48, 112])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_non_finite_rows_leave_the_others(value, K):
+    """One row of x and one of w that are not finite: every other result keeps its
+    bits, also those of the same 16 x 16 block."""
+    g = torch.Generator(device=_dev()).manual_seed(8)
+    x = torch.randn(300, K, generator=g, device=_dev())
+    w = torch.randn(264, K, generator=g, device=_dev())
+    clean = _linear(x, w)
+    x[37, K // 2] = value
+    w[130, 5] = value
+    y = _linear(x, w)
+    assert not torch.isfinite(y[37]).any() and not torch.isfinite(y[:, 130]).any()
+    y[37], y[:, 130] = clean[37], clean[:, 130]
+    assert torch.equal(y, clean)
