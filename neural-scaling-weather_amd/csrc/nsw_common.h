@@ -156,10 +156,19 @@ __device__ __forceinline__ float rows4_max(float x) {
   return fmaxf(c, d);
 }
 
-// Maximum over the four lanes of a quad, on every lane.
-__device__ __forceinline__ float quad_max(float x) {
-  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xf, 0xf, false)));
-  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0x4E, 0xf, 0xf, false)));
+// Second smallest of the four values of a quad's lanes (the smallest where the
+// others are infinite), on every lane.
+__device__ __forceinline__ float quad_second_min(float x) {
+  auto swap1 = [](float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false));
+  };
+  auto swap2 = [](float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, false));
+  };
+  const float y = swap1(x);
+  const float lo = fminf(x, y), hi = fmaxf(x, y), lo2 = swap2(lo), hi2 = swap2(hi);
+  const float second = fminf(fmaxf(lo, lo2), fminf(hi, hi2));
+  return second < INFINITY ? second : fminf(lo, lo2);
 }
 
 // ------------------------------------------- direct-to-LDS copies, waits ----

@@ -70,15 +70,26 @@ typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 // fp32 operands run on the 16-bit matrix instructions, split into two scaled
 // fp16 parts (three products) from this K on and into three bf16 parts (six
-// products) below it.  v_mfma_f32_16x16x4_f32 has 1/16 of their rate; both forms
-// are also closer to the 64-bit result than it was, because a sum takes K / 32
-// x 3 or x 6 roundings instead of K.  Relative error (2-norm) of x . w^T, x
-// N(0, 1), w N(0, 0.02): fp32 instruction / three parts / two parts
-//   K = 112: 4.8e-8 (128) / 4.3e-8 / 4.0e-8    K = 1024: 3.2e-7 / 2.7e-7 / 2.0e-7
-//   K = 192: 7.4e-8 / 6.1e-8 / 5.1e-8          K = 4096: 9.0e-7 / 7.9e-7 / 5.6e-7
-// Below K = 128 the parts' own rounding would be as large as the sum's.  Time
-// (64800 rows, bias): N 3072, K 1024 2853 / 1991 / 1206 us; N 1024, K 4096
-// 3694 / 2620 / 1488 us (365 TFLOP/s of fp32 work, 1.1 PFLOP/s of fp16).
+// products) below it; values that two fp16 parts do not hold are looked for one by
+// one (mainloop_split2).  v_mfma_f32_16x16x4_f32 has 1/16 of their rate; on normal
+// rows both forms are also closer to the 64-bit result than it was, because a sum
+// takes K / 32 x 3 or x 6 roundings instead of K.  Relative error (2-norm) of x .
+// w^T, x N(0, 1), w N(0, 0.02): fp32 instruction / three parts / two parts
+//   K =   32: 1.0e-7 / 3.8e-8 / 8.8e-8       K =  192: 2.5e-7 / 2.0e-7 / 1.6e-7
+//   K =   96: 1.8e-7 / 1.3e-7 / 1.2e-7       K = 1024: 5.7e-7 / 4.8e-7 / 3.6e-7
+//   K =  128: 2.0e-7 / 1.6e-7 / 1.4e-7       K = 4096: 1.2e-6 / 1.0e-6 / 7.1e-7
+// Below K = 128 three parts are as close or closer and mostly faster (us, three /
+// two: 129600 x 128, K 32 17.6 / 25.8; 16200 x 192, K 96 11.8 / 13.7; 64800 x 384, K
+// 112 46.8 / 59.5; 64800 x 1024, K 96 101.9 / 96.3).
+// Time (us, 64800 rows, no bias), N 3072, K 1024 / N 1024, K 4096:
+//   fp32 instruction                                        2829 / 3674
+//   two parts, values not looked at                         1111 / 1430
+//   normal rows                                             1256 / 1659
+//   a column 1e4 times the others                           1605 / 2119
+//   half the values zero                                    1629 / 1996
+//   values of any size (three parts from the first stage)   1882 / 2394
+//   GELU(2 x - 2)                                           2212 / 2491
+//   a row that is not finite                                1322 / 1870
 constexpr int SPLIT2_MIN_K = 128;
 
 // bf16 256 x 256 tiles run mainloop_256.
@@ -306,17 +317,59 @@ __device__ __forceinline__ Split3 split3(const u32x4& a, const u32x4& b) {
 }
 
 // Eight fp32 values times a power of two as the sums of two fp16: h = fp16(x s),
-// l = fp16(x s - h), the difference exact.  h + l is within 2^-23 of x s.
-__device__ __forceinline__ void split2(const u32x4& a, const u32x4& b, float sc, u32x4& h, u32x4& l) {
+// l = fp16(x s - h), the difference exact.  h + l is within 2^-23 of |x s|, or
+// 2^-25 where that is larger, up to |x s| = SPLIT2_MAX.
+constexpr float SPLIT2_MAX = 65504.f;
+__device__ __forceinline__ void split2(const f32x4& a, const f32x4& b, float sc, u32x4& h, u32x4& l) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const float x0 = __builtin_bit_cast(float, e < 2 ? a[2 * e] : b[2 * e - 4]);
-    const float x1 = __builtin_bit_cast(float, e < 2 ? a[2 * e + 1] : b[2 * e - 3]);
+    const float x0 = e < 2 ? a[2 * e] : b[2 * e - 4], x1 = e < 2 ? a[2 * e + 1] : b[2 * e - 3];
     const f16x2 hp = __builtin_convertvector((f32x2{x0 * sc, x1 * sc}), f16x2);
     h[e] = __builtin_bit_cast(uint32_t, hp);
     l[e] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{__builtin_fmaf(x0, sc, -(float)hp[0]),
                                                                        __builtin_fmaf(x1, sc, -(float)hp[1])}), f16x2));
   }
+}
+
+// Lanes that hold a magnitude |x s| below lo or above SPLIT2_MAX (NaN does not
+// count).  The three-input forms as such: fminf and fmaxf put a canonicalising
+// instruction before each value and cost 20% of the GEMM's time.
+__device__ __forceinline__ uint64_t split2_outside(const f32x4& a, const f32x4& b, float sc, float lo) {
+  float mn = fabsf(a[0]), mx = mn;
+  auto min3 = [&](float x, float y) { asm("v_min3_f32 %0, |%1|, |%2|, %0" : "+v"(mn) : "v"(x), "v"(y)); };
+  auto max3 = [&](float x, float y) { asm("v_max3_f32 %0, |%1|, |%2|, %0" : "+v"(mx) : "v"(x), "v"(y)); };
+  min3(a[1], a[2]);
+  max3(a[1], a[2]);
+  min3(a[3], b[0]);
+  max3(a[3], b[0]);
+  min3(b[1], b[2]);
+  max3(b[1], b[2]);
+  min3(b[3], b[3]);
+  max3(b[3], b[3]);
+  return __ballot(mn * sc < lo) | __ballot(mx * sc > SPLIT2_MAX);
+}
+
+// Whether two parts hold x at scale s.
+__device__ __forceinline__ bool split2_holds(float x, float s, float lo) {
+  const float m = fabsf(x * s);
+  return x == 0.f || (m >= lo && m <= SPLIT2_MAX);
+}
+
+// Scale of a row from the eight values that each lane of its quad holds: takes
+// the second smallest of the four lanes' largest magnitudes to [2^11, 2^12), which
+// leaves 2^4 above it and 2^15 to 2^17 below.  (Units listed of 256 rows, normal K
+// = 1024 / GELU of normal values K = 4096 / a Student t of 3 degrees K = 1024:
+// smallest to 2^12 1 / 961 / 155, to 2^11 1 / 11 / 24; second smallest to 2^11 2 /
+// 9 / 6, to 2^10 7 / 21 / 8; largest to 2^10 9 / 35 / 14, and that follows
+// outliers.)  0 while every value is zero.
+__device__ __forceinline__ float split2_scale(const f32x4& a, const f32x4& b) {
+  float m = 0.f;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) m = fmaxf(m, fmaxf(fabsf(a[e]), fabsf(b[e])));
+  m = quad_second_min(m == 0.f ? INFINITY : m);
+  int ex = (int)(__builtin_bit_cast(uint32_t, m) >> 23) - 127;   // 2^ex <= m < 2^(ex + 1)
+  ex = ex < -115 ? -115 : ex;
+  return m == INFINITY ? 0.f : __builtin_bit_cast(float, (uint32_t)(11 - ex + 127) << 23);
 }
 
 // acc += w x of one block from the operands' three parts, smallest products
@@ -440,6 +493,150 @@ __device__ __forceinline__ void mainloop_ring(char* smem, const bf16* __restrict
   }
 }
 
+// Units (16 rows x the 32 k of a stage) with a value that two fp16 parts do not
+// hold (mainloop_split2).  Rows count the tile's x rows, then its w rows.  The list
+// takes three quarters of a stage's units, so that it does not fit the first stage
+// of a tile that has such values everywhere (with all 32 of a 256 x 256 tile listed
+// and added, that tile took 2500 us for 64800 x 3072 x 1024 instead of 1880).
+template <class TC> constexpr int split2_list = (TC::BM + TC::BN) / 16 * 3 / 4;
+constexpr int SPLIT2_LIST = split2_list<BigTile>;
+struct Split2List {
+  int n;                  // units found; those past split2_list are not listed
+  int stop;               // first stage with a unit that is not listed
+  int row[SPLIT2_LIST];   // first row; SPLIT2_ONE + the row of a single small value
+  int k[SPLIT2_LIST];
+};
+constexpr int SPLIT2_ONE = 1 << 16;
+
+// Single small values below k end, whose parts are in the sums: each is at most
+// 2^-25 short, so a result of its row at most 2^-25 SPLIT2_MAX < 2^-9 (all scaled).
+// Returns the entries (bits) with a result of this wave that is not 2^20 times what
+// the row's small values may take from it; what their parts are short of is to be
+// added (normal rows, K = 1024: 5e-4 of the entries and results' blocks).  Results
+// below 4 become NaN, which redo_nonfinite forms again: a product of a subnormal part
+// takes part in the instruction's alignment as if the part were 2^-14, which may
+// take 2^-22 from the others'.  Rows of x or of w that are zero throughout (sh:
+// exponents of the rows' scales, 127 there) are left alone.
+template <class TC>
+__device__ __forceinline__ uint32_t check_small(const Split2List& list, const int* sh, int end,
+                                                f32x4 (&acc)[TC::NB][TC::MB], int wave, int lane) {
+  constexpr int NB = TC::NB, MB = TC::MB;
+  static_assert(SPLIT2_LIST <= 32, "an entry is a bit");
+  const int frow = lane & 15, fg = lane >> 4;
+  const int n = __builtin_amdgcn_readfirstlane(list.n < split2_list<TC> ? list.n : split2_list<TC>);
+  uint32_t add = 0;
+#pragma unroll 1
+  for (int i = 0; i < n; ++i) {
+    int row = __builtin_amdgcn_readfirstlane(list.row[i]);
+    if (row < SPLIT2_ONE || __builtin_amdgcn_readfirstlane(list.k[i]) >= end) continue;
+    const float least = 0x1p11f * (float)__popcll(__ballot(lane < n && list.row[lane < n ? lane : 0] == row));
+    row -= SPLIT2_ONE;
+    const bool isx = row < TC::BM;
+    const int r = isx ? row - (wave / TC::WGN) * TC::WTM : row - TC::BM - (wave % TC::WGN) * TC::WTN;   // of this wave
+    if (r < 0 || r >= (isx ? TC::WTM : TC::WTN)) continue;
+    const bool mine = isx ? frow == (r & 15) : fg == ((r >> 2) & 3);
+    bool low = false;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb) {
+        if ((isx ? mb : nb) != r >> 4) continue;
+        const int xr = (wave / TC::WGN) * TC::WTM + mb * 16 + frow, wr = TC::BM + (wave % TC::WGN) * TC::WTN + nb * 16 + 4 * fg;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float m = fabsf(acc[nb][mb][c]);
+          if (mine && (isx || c == (r & 3)) && m < least && sh[xr] != 127 && sh[wr + c] != 127) {
+            low = true;
+            if (m < 4.f) acc[nb][mb][c] = __builtin_nanf("");
+          }
+        }
+      }
+    if (__ballot(low) != 0) add |= 1u << i;
+  }
+  return add;
+}
+
+// What the parts of a value outside the window are short of at scale s: all of it
+// where it was given none (not small), else what they round away.
+__device__ __forceinline__ float split2_rest(float x, float s, bool small) {
+  const float v = x * s;
+  if (!small || fabsf(v) <= 0x1p-25f) return x;
+  const _Float16 h = (_Float16)v;
+  const float d = v - (float)h;
+  return __builtin_amdgcn_ldexpf(d - (float)(_Float16)d, 127 - (int)(__builtin_bit_cast(uint32_t, s) >> 23));
+}
+
+// What the parts of the listed units below k end are short of (of single small
+// values: those in `small`), times the other operand, with the fp32 matrix
+// instruction.  A pair of two values without parts counts once, for the unit of x;
+// else the other operand's values count whole.  sh: exponents of the rows' scales.
+// The sums of a unit pass through LDS (buf, a KB a block), so that they are formed
+// in one rolled loop: added to the accumulators where they are formed, the
+// accumulators spilled.  2 us a unit of x and 5 us a unit of w of a 256 x 256 tile,
+// a quarter of that for the single small values that need nothing.
+template <class TC>
+__device__ __forceinline__ void add_outside(const Split2List& list, const int* sh, char* buf, const float* __restrict__ X,
+                                            const float* __restrict__ Wt, int M, int N, int K, int m0, int n0, int end,
+                                            float lo, uint32_t small, f32x4 (&acc)[TC::NB][TC::MB], int wave, int lane) {
+  constexpr int NB = TC::NB, MB = TC::MB;
+  const int frow = lane & 15, fg = lane >> 4;
+  const int xw = (wave / TC::WGN) * TC::WTM, ww = (wave % TC::WGN) * TC::WTN;   // this wave's first x and w rows
+  const int n = __builtin_amdgcn_readfirstlane(list.n < split2_list<TC> ? list.n : split2_list<TC>);
+#pragma unroll 1
+  for (int i = 0; i < n; ++i) {
+    int row = __builtin_amdgcn_readfirstlane(list.row[i]);
+    const int k = __builtin_amdgcn_readfirstlane(list.k[i]);
+    const bool one = row >= SPLIT2_ONE;
+    row &= SPLIT2_ONE - 1;
+    const bool isx = row < TC::BM;
+    const int blk = (isx ? row - xw : row - TC::BM - ww) >> 4;      // this wave's row block
+    if (k >= end || (one && (small >> i & 1) == 0) || blk < 0 || blk >= (isx ? MB : NB)) continue;
+    f32x4* sum = reinterpret_cast<f32x4*>(buf) + wave * (MB > NB ? MB : NB) * 64 + lane;
+    // lane (i, g): k 4g..4g+3 and 16+4g..+3 of row i of a block (the second half
+    // of the last stage may lie past K: zero)
+    auto load = [&](bool ofx, int b, f32x4 (&v)[2]) {
+      const int g = ofx ? m0 + xw + b * 16 + frow : n0 + ww + b * 16 + frow, rows = ofx ? M : N;
+      const float* p = (ofx ? X : Wt) + (int64_t)(g < rows ? g : rows - 1) * K + k + 4 * fg;
+      v[0] = *reinterpret_cast<const f32x4*>(p);
+      v[1] = k + 16 < K ? *reinterpret_cast<const f32x4*>(p + 16) : f32x4{0.f, 0.f, 0.f, 0.f};
+    };
+    auto scale = [&](bool ofx, int b) {
+      return __builtin_amdgcn_ldexpf(1.f, -sh[(ofx ? xw : TC::BM + ww) + b * 16 + frow]);
+    };
+    constexpr int G = MB < NB ? MB : NB;      // blocks of the other operand whose loads are in flight together
+    f32x4 u[2];
+    load(isx, blk, u);
+    const float us = scale(isx, blk);
+#pragma unroll 1
+    for (int b = 0; b < (isx ? NB : MB); b += G) {
+      f32x4 o[G][2];
+#pragma unroll
+      for (int j = 0; j < G; ++j) load(!isx, b + j, o[j]);
+#pragma unroll
+      for (int j = 0; j < G; ++j) {
+        const float os = scale(!isx, b + j);
+        // the other unit may have values without parts itself
+        const int orow = isx ? TC::BM + ww + (b + j) * 16 : xw + (b + j) * 16, l = lane < n ? lane : 0;
+        const bool both = (one || !isx) && __ballot(lane < n && list.row[l] == orow && list.k[l] == k) != 0;
+        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          float r = u[e >> 2][e & 3], q = o[j][e >> 2][e & 3];
+          r = split2_holds(r, us, lo) ? 0.f : split2_rest(r, us, one);
+          if (both && !split2_holds(q, os, lo)) q = 0.f;
+          c = __builtin_amdgcn_mfma_f32_16x16x4f32(isx ? q : r, isx ? r : q, c, 0, 0, 0);
+        }
+        sum[(b + j) * 64] = c;
+      }
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        if ((isx ? mb : nb) == blk) acc[nb][mb] += sum[(isx ? nb : mb) * 64];
+  }
+}
+
 // fp32 main loop on two fp16 parts of each operand (rows scaled by powers of
 // two), three products.  A stage is 32 k: one step of the 16-bit matrix
 // instructions, lane group g taking k 4g..4g+3 and 16+4g..+3 of both operands.
@@ -450,42 +647,49 @@ __device__ __forceinline__ void mainloop_ring(char* smem, const bf16* __restrict
 // wave that reads it: the wave that copied 16 stage rows splits them in place,
 // the h parts into the chunk of k 4c.. and the l parts into that of 16+4c...
 //
-// A ring of NST slots.  In stage s the wave splits its rows of stage s + 1 under
+// A ring of two slots.  In stage s the wave splits its rows of stage s + 1 under
 // the MFMAs before row block BARB; the stage's one barrier stands there, once
 // every fragment of the stage is in registers: past it the next stage's first
-// fragments are read, and the copies of stage s + NST start into the slot just
+// fragments are read, and the copies of stage s + 2 start into the slot just
 // read.  Issued in one go the copies hold every wave for the ~1000 cycles that
 // the CU's address path takes for 64 KB, so they are spread, and they carry no
 // condition (past the end they re-read the last stage into a slot whose values
 // are not used).
 //
-// A row's scale takes the largest magnitude of its first 32 k to [32, 64).  The
-// row's own maximum is no smaller, so what fp16 rounds away below 2^-24 is
-// under 2^-29 of it, and values up to 2^10 times the sampled maximum fit;
-// beyond that the results are not finite and the tile is formed again from
-// three bf16 parts.  A row whose first 32 k are zero is scanned; one that is
-// zero throughout gets scale 1.
+// Range.  Two parts hold a scaled magnitude between lo and SPLIT2_MAX to 2^-25 /
+// lo of itself or better, and zero.  Every value is looked at before it is split.
+// The unit of one outside goes on a list.  A single small value keeps its parts;
+// the results of its row are looked at in the end, and what the parts are short of
+// is added where it matters (check_small, add_outside).  Otherwise the values
+// outside get zero parts and their products are added in the end.  A product keeps within (K / 8 + 4) 2^-24 of itself
+// whatever else its rows hold, a quarter of what K fp32 additions may lose: lo = 8 /
+// K costs each of the two values K / 16 2^-24, and leaving out the product of the l
+// parts 4 2^-24.  lo is no lower than 2^-6, so that a value is never further off
+// than 2^-19.  Rows of normal values put about 5 K / 1024 units of a 256 x 256 tile
+// on the list, nearly all with one small value.  A tile whose list is full leaves
+// the loop before the stage that did not fit; the caller goes on from that stage
+// (the return value) on three parts.
+//
+// A row's scale is set at its first stage that is not zero throughout
+// (split2_scale; until then it is 0).
 template <class TC>
-__device__ __forceinline__ void mainloop_split2(char* smem, const float* __restrict__ X, const float* __restrict__ Wt,
-                                                int M, int N, int K, int m0, int n0, f32x4 (&acc)[TC::NB][TC::MB],
-                                                int wave, int lane) {
-  constexpr int NB = TC::NB, MB = TC::MB, NST = TC::NST;
+__device__ __forceinline__ int mainloop_split2(char* smem, Split2List& list, const float* __restrict__ X,
+                                               const float* __restrict__ Wt, int M, int N, int K, int m0, int n0,
+                                               f32x4 (&acc)[TC::NB][TC::MB], int wave, int lane) {
+  constexpr int NB = TC::NB, MB = TC::MB;
   constexpr int BARB = MB > 2 ? MB - 2 : 1;      // row block before which the barrier stands
   using Copy = StageCopy<float, TC>;
   constexpr int NC = Copy::NC, NU = NC / 2;      // copies, 16-row units to split
   constexpr int NC1 = NC * 3 / 4;                // copies issued past the barrier; the others in the next stage
   constexpr int SPLB = BARB > 2 ? 2 : BARB - 1;  // first row block with splits
+  static_assert(TC::NST == 2, "a ring of two slots");
   static_assert(Copy::CX % 2 == 0 && Copy::CW % 2 == 0, "units of 16 rows of one operand");
   Copy cp;
   cp.init(smem, X, Wt, M, N, K, m0, n0, wave, lane);
   const int nst = cp.nst;
-  // deep rings copy stages that exist only (short sums end before their ring
-  // is full; the branch matters less than draining copies nobody needs)
-  constexpr bool COND = NST > 2;
-#pragma unroll
-  for (int s = 0; s < NST - 1; ++s)
-    if (!COND || s < nst) cp.copy(s < nst ? s : nst - 1, s, 0, NC);
-  if (!COND || NST - 1 < nst) cp.copy(NST - 1 < nst ? NST - 1 : nst - 1, NST - 1, 0, NC1);
+  const float lo = fmaxf(8.f / (float)K, 0x1p-6f);
+  cp.copy(0, 0, 0, NC);
+  cp.copy(nst > 1 ? 1 : 0, 1, 0, NC1);
   // this lane's row of a unit and its chunk pair (c, c + 4): any 16 lanes
   // cover four rows whose pairs lie in distinct banks
   const int li = lane >> 2, lc = lane & 3;
@@ -493,36 +697,65 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
   const int uoff = urow * ROWB + (lc ^ row_swizzle(urow)) * 16;   // chunk c; chunk c + 4 is at ^ 64
   auto unit = [&](int u) { return (u < Copy::CX / 2 ? 0 : TC::BM * ROWB) + cp.row(2 * u) * ROWB + uoff; };
   float sc[NU];
-  if (!COND || NST <= nst) wait_copies<(NST - 2) * NC + NC1>();
-  else wait_copies();
-#pragma unroll
-  for (int u = 0; u < NU; ++u) {
-    char* p = smem + unit(u);
-    char* q = smem + (unit(u) ^ 64);
-    const u32x4 a = *reinterpret_cast<const u32x4*>(p), b = *reinterpret_cast<const u32x4*>(q);
-    float m = 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      m = fmaxf(m, fmaxf(fabsf(__builtin_bit_cast(float, a[e])), fabsf(__builtin_bit_cast(float, b[e]))));
-    m = quad_max(m);
-    if (__ballot(m == 0.f) != 0) {
-      const int r = cp.row(2 * u) + urow;
-      const float* g = u < Copy::CX / 2 ? X + (int64_t)(m0 + r < M ? m0 + r : M - 1) * K
-                                        : Wt + (int64_t)(n0 + r < N ? n0 + r : N - 1) * K;
-      for (int k = 4 * lc; k < K; k += 16) {
-        const f32x4 v = *reinterpret_cast<const f32x4*>(g + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = fmaxf(m, fabsf(v[e]));
-      }
-      m = quad_max(m);
+  // looks at unit u of stage s: a, b stay what is to be split
+  auto look = [&](int u, int s, f32x4& a, f32x4& b) {
+    if (__builtin_expect(split2_outside(a, b, sc[u], lo) == 0, 1)) return;
+    // a value outside the window, or a zero
+    if (__ballot(sc[u] == 0.f) != 0) {
+      const float t = split2_scale(a, b);
+      if (sc[u] == 0.f) sc[u] = t;
     }
-    int ex = (int)(__builtin_bit_cast(uint32_t, m) >> 23) - 127;   // 2^ex <= m < 2^(ex + 1)
-    ex = m == 0.f ? 5 : ex < -120 ? -120 : ex > 120 ? 120 : ex;
-    sc[u] = __builtin_bit_cast(float, (uint32_t)(5 - ex + 127) << 23);
+    const int row = (u < Copy::CX / 2 ? 0 : TC::BM) + cp.row(2 * u);
+    const bool stored = u < Copy::CX / 2 ? m0 + row + urow < M : n0 + row + urow - TC::BM < N;   // not a repeated last row
+    int count = 0;
+    bool large = false;
+    auto see = [&](float x) {
+      count += !split2_holds(x, sc[u], lo);
+      large |= !(fabsf(x * sc[u]) <= SPLIT2_MAX);
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      see(a[e]);
+      see(b[e]);
+    }
+    const uint64_t lanes = __ballot(count != 0 && stored);
+    const bool one = __popcll(lanes) == 1 && __ballot(count > 1 || large) == 0;
+    if (!one) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        a[e] = split2_holds(a[e], sc[u], lo) ? a[e] : 0.f;
+        b[e] = split2_holds(b[e], sc[u], lo) ? b[e] : 0.f;
+      }
+    }
+    if (lanes != 0 && s < nst && lane == (one ? __builtin_ctzll(lanes) : 0)) {
+      const int i = __hip_atomic_fetch_add(&list.n, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      if (i < split2_list<TC>) {
+        list.row[i] = one ? SPLIT2_ONE + row + urow : row;
+        list.k[i] = s * 32;
+      } else {
+        __hip_atomic_fetch_min(&list.stop, s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      }
+    }
+  };
+  // the parts of unit u into its slot
+  auto put = [&](int u, char* st, const f32x4& a, const f32x4& b) {
     u32x4 h, l;
     split2(a, b, sc[u], h, l);
-    *reinterpret_cast<u32x4*>(p) = h;
-    *reinterpret_cast<u32x4*>(q) = l;
+    *reinterpret_cast<u32x4*>(st + unit(u)) = h;
+    *reinterpret_cast<u32x4*>(st + (unit(u) ^ 64)) = l;
+  };
+  if (wave == 0 && lane == 0) {
+    list.n = 0;
+    list.stop = 0x7fffffff;
+  }
+  wg_barrier();        // the list is empty before any wave adds to it
+  wait_copies<NC1>();
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    f32x4 a = *reinterpret_cast<const f32x4*>(smem + unit(u)), b = *reinterpret_cast<const f32x4*>(smem + (unit(u) ^ 64));
+    sc[u] = split2_scale(a, b);
+    look(u, 0, a, b);
+    put(u, smem, a, b);
   }
   wg_barrier();
   const int frow = lane & 15, fg = lane >> 4;
@@ -537,45 +770,47 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
   for (int nb = 0; nb < NB; ++nb) load(smem, wrow + nb * 16, ws[nb]);
   load(smem, xrow, xs[0]);
   load(smem, xrow + 16, xs[1]);
-  int slot = 0;
-  for (int s = 0; s < nst; ++s) {
-    const int nslot = slot + 1 == NST ? 0 : slot + 1, pslot = slot == 0 ? NST - 1 : slot - 1;
-    char* st = smem + slot * TC::SLOT;
-    char* sn = smem + nslot * TC::SLOT;
-    // the rest of stage s + NST - 1 here, most of stage s + NST past the barrier
-    const int c1 = s + NST - 1, c2 = s + NST;
-    if (!COND || c1 < nst) cp.copy(c1 < nst ? c1 : nst - 1, pslot, NC1, NC);
+  // the first stage not to be run; a wave that is a stage ahead may have put a
+  // later stage into list.stop by the time another reads it, never this one
+  auto stopped = [&](int s) { return __builtin_amdgcn_readfirstlane(list.stop) <= s; };
+  int s = 0;
+  for (bool stop = stopped(0); s < nst && !stop; ++s) {
+    char* st = smem + (s & 1) * TC::SLOT;
+    char* sn = smem + ((s + 1) & 1) * TC::SLOT;
+    // the rest of stage s + 1 here, most of stage s + 2 past the barrier
+    const int c1 = s + 1 < nst ? s + 1 : nst - 1, c2 = s + 2 < nst ? s + 2 : nst - 1;
+    cp.copy(c1, (s + 1) & 1, NC1, NC);
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       if (mb == BARB) {
         wg_barrier();
+        stop = stopped(s + 1);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) load(sn, wrow + nb * 16, wn[nb]);
       }
       if (mb >= BARB) {
         constexpr int L = MB - BARB;                 // row blocks past the barrier
-        if (!COND || c2 < nst) cp.copy(c2 < nst ? c2 : nst - 1, slot, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
+        cp.copy(c2, s & 1, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
       }
       if (mb + 2 < MB) load(st, xrow + (mb + 2) * 16, xs[(mb + 2) % 3]);
       // the units of the next stage, split ahead of the barrier
-      if (mb == SPLB) {
-        if (!COND || c1 < nst) wait_copies<(NST - 2) * NC>();
-        else wait_copies();
-      }
+      if (mb == SPLB) wait_copies();
+      f32x4 ua[NU], ub[NU];
 #pragma unroll
       for (int u = 0; u < NU; ++u) {
         if (mb != SPLB + u * (BARB - SPLB) / NU) continue;
-        char* p = sn + unit(u);
-        char* q = sn + (unit(u) ^ 64);
-        const u32x4 a = *reinterpret_cast<const u32x4*>(p), b = *reinterpret_cast<const u32x4*>(q);
-        u32x4 h, l;
-        split2(a, b, sc[u], h, l);
-        *reinterpret_cast<u32x4*>(p) = h;
-        *reinterpret_cast<u32x4*>(q) = l;
+        ua[u] = *reinterpret_cast<const f32x4*>(sn + unit(u));
+        ub[u] = *reinterpret_cast<const f32x4*>(sn + (unit(u) ^ 64));
       }
       const f16x8 (&x)[2] = xs[mb % 3];
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) mfma_f16(acc[nb][mb], ws[nb][1], x[0]);
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        if (mb != SPLB + u * (BARB - SPLB) / NU) continue;
+        look(u, s + 1, ua[u], ub[u]);
+        put(u, sn, ua[u], ub[u]);
+      }
 #pragma unroll
       for (int nb = 0; nb < NB; ++nb) mfma_f16(acc[nb][mb], ws[nb][0], x[1]);
 #pragma unroll
@@ -587,16 +822,17 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
     for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
       for (int i = 0; i < 2; ++i) ws[nb][i] = wn[nb][i];
-    slot = nslot;
   }
   wait_copies();       // those past the last stage
   wg_barrier();        // the ring is no longer read
-  // scale back: the rows' exponents pass through LDS
+  // scale back: the rows' exponents pass through LDS (a row without a scale is
+  // zero throughout)
   int* sh = reinterpret_cast<int*>(smem);
 #pragma unroll
   for (int u = 0; u < NU; ++u)
     if (lc == 0) sh[(u < Copy::CX / 2 ? 0 : TC::BM) + cp.row(2 * u) + urow] = 127 - (int)(__builtin_bit_cast(uint32_t, sc[u]) >> 23);
   wg_barrier();
+  const uint32_t small = check_small<TC>(list, sh, s * 32, acc, wave, lane);
   int ex[MB];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) ex[mb] = sh[xrow + mb * 16];
@@ -609,19 +845,23 @@ __device__ __forceinline__ void mainloop_split2(char* smem, const float* __restr
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) acc[nb][mb][r] = __builtin_amdgcn_ldexpf(acc[nb][mb][r], e[r] + ex[mb]);
   }
+  add_outside<TC>(list, sh, smem + 4096, X, Wt, M, N, K, m0, n0, s * 32, lo, small, acc, wave, lane);
+  wg_barrier();        // the exponents are no longer read
+  return s;
 }
 
 // fp32 main loop on three bf16 parts of each operand, which hold any fp32
 // value: of the nine products the six of weight >= 2^-16, smallest first, and
 // the three dropped are below 2^-24 of the product, as fp32's own rounding.
-// For short K (gemm_kernel) and tiles that two scaled fp16 parts do not hold.
+// For short K (gemm_kernel) and, from stage `first` on, tiles that two scaled fp16
+// parts do not hold.
 // Stages, barrier and copies as mainloop_split2, but the parts do not fit in
 // place, so every wave splits the fragments it reads: w block nb + 1 under the
 // MFMAs of (nb, mb 0), x block mb + 1 under those of block mb.
 template <class TC>
 __device__ __forceinline__ void mainloop_split3(char* smem, const float* __restrict__ X, const float* __restrict__ Wt,
                                                 int M, int N, int K, int m0, int n0, f32x4 (&acc)[TC::NB][TC::MB],
-                                                int wave, int lane) {
+                                                int wave, int lane, int first) {
   constexpr int NB = TC::NB, MB = TC::MB;
   constexpr int BARB = MB > 2 ? MB - 2 : 1;      // row block before which the barrier stands
   using Copy = StageCopy<float, TC>;
@@ -629,8 +869,9 @@ __device__ __forceinline__ void mainloop_split3(char* smem, const float* __restr
   Copy cp;
   cp.init(smem, X, Wt, M, N, K, m0, n0, wave, lane);
   const int nst = cp.nst;
-  cp.copy(0, 0, 0, NC);
-  cp.copy(nst > 1 ? 1 : 0, 1, 0, NC1);
+  if (first >= nst) return;
+  cp.copy(first, 0, 0, NC);
+  cp.copy(first + 1 < nst ? first + 1 : first, 1, 0, NC1);
   const int frow = lane & 15, fg = lane >> 4;
   const int xrow = (wave / TC::WGN) * TC::WTM + frow;             // x rows of this wave (B operand)
   const int wrow = TC::BM + (wave % TC::WGN) * TC::WTN + frow;    // w rows of this wave (A operand)
@@ -646,15 +887,16 @@ __device__ __forceinline__ void mainloop_split3(char* smem, const float* __restr
   load(smem, xrow, rx_[0]);
   load(smem, xrow + 16, rx_[1]);
   Split3 ws[NB], xs = split3(rx_[0][0], rx_[0][1]), w0 = split3(rw_[0][0], rw_[0][1]), xn;
-  for (int s = 0; s < nst; ++s) {
-    const char* st = smem + (s & 1) * TC::SLOT;
-    const char* sn = smem + ((s + 1) & 1) * TC::SLOT;
+  for (int s = first; s < nst; ++s) {
+    const int slot = (s - first) & 1;
+    const char* st = smem + slot * TC::SLOT;
+    const char* sn = smem + (slot ^ 1) * TC::SLOT;
     const int c1 = s + 1 < nst ? s + 1 : nst - 1, c2 = s + 2 < nst ? s + 2 : nst - 1;
     if (MB > 2) load(st, xrow + 32, rx_[0]);
     ws[0] = w0;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      cp.copy(c1, (s + 1) & 1, NC1 + nb * (NC - NC1) / NB, NC1 + (nb + 1) * (NC - NC1) / NB);
+      cp.copy(c1, slot ^ 1, NC1 + nb * (NC - NC1) / NB, NC1 + (nb + 1) * (NC - NC1) / NB);
       mul_parts(acc[nb][0], ws[nb], xs);
       if (nb + 1 < NB) ws[nb + 1] = split3(rw_[nb + 1][0], rw_[nb + 1][1]);
       else xn = split3(rx_[1][0], rx_[1][1]);
@@ -673,7 +915,7 @@ __device__ __forceinline__ void mainloop_split3(char* smem, const float* __restr
       }
       if (mb >= BARB) {
         constexpr int L = MB - BARB;             // row blocks past the barrier
-        cp.copy(c2, s & 1, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
+        cp.copy(c2, slot, (mb - BARB) * NC1 / L, (mb - BARB + 1) * NC1 / L);
       }
       if (mb + 2 < MB) load(st, xrow + (mb + 2) * 16, rx_[mb & 1]);
       if (mb == BARB) {
@@ -884,23 +1126,15 @@ __global__ __launch_bounds__(TC::NW * 64, TC::MINW) void gemm_kernel(const T* __
     } else if constexpr (sizeof(T) == 2) {
       mainloop_ring<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
     } else {
-      bool three = K < SPLIT2_MIN_K;
-      if (!three) {
-        __shared__ int redo;
-        if (threadIdx.x == 0) redo = 0;     // before the main loop's barriers
-        mainloop_split2<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
-        if (any_nonfinite<TC>(acc)) redo = 1;
-        wg_barrier();
-        three = redo != 0;
+      // on two fp16 parts as long as they hold the tile's values, then on three
+      // bf16 parts
+      int stage = 0;
+      if (K >= SPLIT2_MIN_K) {
+        __shared__ Split2List list;
+        stage = mainloop_split2<TC>(smem, list, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
       }
-      if (three) {
-#pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-          for (int j = 0; j < MB; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        mainloop_split3<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0);
-        redo_nonfinite<TC>(smem, X, Wt, M, N, K, m0 + wm * WTM, n0 + wn * WTN, acc, wave, lane0);
-      }
+      mainloop_split3<TC>(smem, X, Wt, M, N, K, m0, n0, acc, wave, lane0, stage);
+      redo_nonfinite<TC>(smem, X, Wt, M, N, K, m0 + wm * WTM, n0 + wn * WTN, acc, wave, lane0);
     }
   }
   NSW_STAMP(ts[2]);
