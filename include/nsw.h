@@ -167,6 +167,12 @@ int nsw_proj_reverse_residual(const void* o, const void* wproj, const void* bpro
                               int64_t W, int64_t C, int64_t ws0, int64_t ws1, int64_t s0,
                               int64_t s1, int dtype, void* stream);
 
+/* Rows of the tile that a product x[M,K] . w[N,K]^T runs on (256 for the large
+ * ones; fewer where those would leave compute units idle), with an epilogue that
+ * stores rows through a map or writes row sums of squares (row_epilogue != 0) or
+ * without.  Host only; 0 for sizes or dtypes that there are none for. */
+int nsw_gemm_tile_rows(int64_t M, int64_t N, int64_t K, int row_epilogue, int dtype);
+
 /* Number of partial sums per row that nsw_proj_reverse_residual_sumsq writes
  * for rows of C elements: one per 512 bytes of row, ceil(C * esize / 512). */
 int64_t nsw_row_sumsq_parts(int64_t C, int dtype);

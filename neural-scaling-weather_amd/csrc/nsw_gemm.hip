@@ -259,6 +259,17 @@ extern "C" int nsw_proj_reverse_residual(const void* o, const void* wproj, const
   return gemm_proj_scatter(o, wproj, bproj, skip, y, B, T, H, W, C, ws0, ws1, s0, s1, dtype, stream, nullptr);
 }
 
+extern "C" int nsw_gemm_tile_rows(int64_t M, int64_t N, int64_t K, int row_epilogue, int dtype) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  auto rows = [](TileSize t, int big, int mid, int small) { return t == TILE_BIG ? big : t == TILE_MID ? mid : small; };
+  const EpiArgs ea{};
+  if (dtype == NSW_DTYPE_F32)
+    return rows(pick_tile<float, EPI_NONE>(M, N, K, ea), BigTile::BM, MidTile::BM, SmallF32Tile::BM);
+  if (dtype != NSW_DTYPE_BF16) return 0;
+  if (row_epilogue) return rows(pick_tile<bf16, EPI_RES_SUMSQ>(M, N, K, ea), BigTile::BM, MidRowTile::BM, SmallRowTile::BM);
+  return rows(pick_tile<bf16, EPI_NONE>(M, N, K, ea), BigTile::BM, MidTile::BM, SmallTile::BM);
+}
+
 extern "C" int64_t nsw_row_sumsq_parts(int64_t C, int dtype) { return C > 0 ? sumsq_parts(C, dtype) : 0; }
 
 extern "C" int nsw_proj_reverse_residual_sumsq(const void* o, const void* wproj, const void* bproj,

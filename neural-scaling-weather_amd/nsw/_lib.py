@@ -90,6 +90,7 @@ SIGNATURES = {
     "nsw_hbm_stream": (_int, [_vp, _vp, _i64, _i64, _vp]),
     "nsw_linear_rowscale": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _f32, _int,
                                    _vp]),
+    "nsw_gemm_tile_rows": (_int, [_i64, _i64, _i64, _int, _int]),
     "nsw_row_sumsq_parts": (_i64, [_i64, _int]),
     "nsw_qkv_projection_rowscale": (_int, [_vp, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _i64, _i64, _i64, _i64, _int,
                                            _vp]),

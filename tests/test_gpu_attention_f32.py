@@ -63,9 +63,10 @@ def test_attention_f32_mask_extremes(L):
     assert _rel(o[:, keep], want[:, keep]) < 1e-5
 
 
-@pytest.mark.parametrize("scale", [0.0, -0.3, 1e-30])
+@pytest.mark.parametrize("scale", [0.0, -0.3, 1e-37, 1e-30])
 def test_attention_f32_scales(scale):
-    """Scales outside the kernel's rule go to the generic kernel, with the shift mask."""
+    """Scales that are not positive or whose -100 / scale is not finite (1e-37) go to
+    the generic kernel, with the shift mask; 1e-30 is the smallest kind that does not."""
     H, W = 18, 36
     qkv = _qkv(4, 162, 64, 9)
     o = nsw.ops.window_attention(qkv, 2, scale, geometry=(H, W, (9, 18), (4, 9), 1))

@@ -164,13 +164,63 @@ def test_split_gemm_non_finite(K):
     assert ((y[keep].double() - want).abs() <= U * (K / 8 + 4) * want).all()
 
 
-# Shapes on both sides of the tile rule (few rows: 64- / 32-row tiles; some
-# hundreds: 128- / 64-row tiles; then 256), with rows and columns that end
+def _tile_rows(M, N, K, dtype, row_epilogue=0):
+    code = _lib.NSW_DTYPE_F32 if dtype == torch.float32 else _lib.NSW_DTYPE_BF16
+    return _lib.lib().nsw_gemm_tile_rows(M, N, K, row_epilogue, code)
+
+
+# The fp32 loops on each tile (64 x 128, 128 x 128, 256 x 256: other waves,
+# copies, splits and barriers), rows and columns that end inside a tile, K with an
+# odd half stage, on three parts (112), two (144, 272) and from one to the other.
+@pytest.mark.parametrize("K", [112, 144, 272])
+@pytest.mark.parametrize("M,N,rows", [(301, 264, 64), (5000, 1160, 128), (8100, 3080, 256)])
+@pytest.mark.parametrize("case", ["normal", "outliers", "singles", "spread", "later", "zero_start", "non_finite"])
+def test_split_gemm_on_each_tile(case, M, N, rows, K):
+    assert _tile_rows(M, N, K, torch.float32) == rows
+    g = torch.Generator(device=_dev()).manual_seed(M + K)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=_dev())
+    x, w = rnd(M, K), 0.02 * rnd(N, K)
+    if case == "outliers":                 # a column of x, one of w: every row block of a stage
+        x[:, 3], w[:, 3] = 1e5, 0
+        w[:, K - 5], x[:, K - 5] = 1e3, 0
+    elif case == "singles":                # two single small values and a large one in most tiles
+        x[::37, 20] = 1e-8
+        w[::67, K - 9] = -1e-9
+        x[11::131, 7] = 3e7
+    elif case == "spread":
+        x *= torch.exp2(torch.randint(-30, 30, (K,), generator=g, device=_dev()).float())
+        w *= torch.exp2(torch.randint(-30, 30, (K,), generator=g, device=_dev()).float())
+    elif case == "later":                  # two parts first, three from a later stage on
+        x[:, K - 20:] *= torch.exp2(torch.randint(-40, 0, (M, 20), generator=g, device=_dev()).float())
+    elif case == "zero_start":
+        x[::3, :40] = 0
+        w[1::3, :K - 3] = 0
+    elif case == "non_finite":
+        x[M - 2, K - 1], w[N - 3, 1] = float("inf"), float("nan")
+        y = _linear(x, w)
+        assert not torch.isfinite(y[M - 2]).any() and torch.isnan(y[:, N - 3]).all()
+        x[M - 2, K - 1], w[N - 3, 1] = 0, 0
+        clean = _linear(x, w)
+        y[M - 2], y[:, N - 3] = clean[M - 2], clean[:, N - 3]
+        # the values were outside the window or not: other rows differ in how one
+        # unit of the tile was listed, by no more than the bound
+        mag = x.double().abs() @ w.double().abs().t()
+        assert ((y.double() - clean.double()).abs() <= 2 * U * (K / 8 + 4) * mag).all()
+    _check(x, w)
+
+
+# Shapes on both sides of the tile rule (64- / 32-row tiles; at 8100 x 1024 rows
+# 128- / 64-row tiles; then 256), with rows and columns that end
 # inside a tile, odd k stages, and every kind of write-out: plain, GELU,
 # residual, the head norm, window maps with row sums, the head's image.
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("H,W,C", [(9, 18, 96), (27, 54, 128), (45, 108, 192), (90, 90, 512)])
+@pytest.mark.parametrize("H,W,C", [(9, 18, 96), (27, 54, 128), (45, 108, 192), (90, 90, 512), (90, 90, 1024),
+                                   (90, 180, 1024)])
 def test_tile_sizes(dtype, H, W, C):
+    f32 = dtype == torch.float32
+    mid, small = C == 1024 and H == W, C < 1024
+    assert _tile_rows(H * W, C, C, dtype) == (64 if small else 128 if mid else 256)
+    assert _tile_rows(H * W, C, C, dtype, 1) == ((64 if f32 else 32) if small else (128 if f32 else 64) if mid else 256)
     g = torch.Generator(device=_dev()).manual_seed(H + C)
     rnd = lambda *s: torch.randn(*s, generator=g, device=_dev()).to(dtype)
     M, hd = H * W, 32
@@ -179,7 +229,7 @@ def test_tile_sizes(dtype, H, W, C):
     w3, b3 = (0.05 * torch.randn(3 * C, C, generator=g, device=_dev())).to(dtype), rnd(3 * C)
     qn, kn = rnd(hd), rnd(hd)
     d = lambda t: t.double()
-    tol = 1e-6 if dtype == torch.float32 else 5e-3     # K <= 512: U sqrt(K) < 1e-6; bf16 store 2^-8 / sqrt(3)
+    tol = 1e-6 if f32 else 5e-3     # U sqrt(K) / 2 <= 1e-6 (a chain of K roundings: U sqrt(K)); bf16 store 2^-8 / sqrt(3)
 
     def close(y, want):
         e = (d(y) - want).norm() / want.norm()
