@@ -354,11 +354,12 @@ __device__ __forceinline__ u32x4 uniform_rsrc(const void* p, uint32_t bytes) {
                (uint32_t)__builtin_amdgcn_readfirstlane((int)r[2]), (uint32_t)__builtin_amdgcn_readfirstlane((int)r[3])};
 }
 
-// 16-byte store from inline asm.  A VALU write to the data VGPRs of a 16-byte
-// store needs 2 wait states after the store on gfx950; the compiler cannot
-// see the store inside the asm, so the s_nop provides them.
+// 16-byte store from inline asm.  The store reads the descriptor 5 wait states
+// after a vector instruction wrote it at the earliest, and a VALU write to the
+// data VGPRs of a 16-byte store needs 2 wait states after the store on gfx950; the
+// compiler cannot see the store inside the asm, so the s_nops provide both.
 __device__ __forceinline__ void store16_asm(const u32x4& rsrc, uint32_t voff, const f32x4& v) {
-  asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen\n\ts_nop 1" : : "v"(v), "v"(voff), "s"(rsrc) : "memory");
+  asm volatile("s_nop 4\n\tbuffer_store_dwordx4 %0, %1, %2, 0 offen\n\ts_nop 1" : : "v"(v), "v"(voff), "s"(rsrc) : "memory");
 }
 
 // One 16-query block of a (window, head) item with head dim 64: K rows and V

@@ -185,7 +185,11 @@ __device__ __forceinline__ u32x4 make_rsrc(const void* p, uint32_t bytes) {
 // Issued as inline asm so that the compiler's wait-count insertion does not
 // see an LDS write in flight (it would otherwise drain all copies before
 // each fragment read); ordering is kept by the explicit vmcnt waits and
-// barriers of the pipeline.  s_nop: M0 write -> LDS-DMA read hazard.
+// barriers of the pipeline.  The copy reads M0 one wait state after its write and
+// its scalar operands 5 after a vector instruction wrote them (here: the
+// v_readfirstlane below, straight before the asm); the compiler sees neither, so the
+// asm waits for both (s_mov_b32 and s_nop 3: 5 states; without, a copy could run
+// with the descriptor that the registers held before).
 // The scalar operands pass through v_readfirstlane, which the compiler drops
 // when they already live in SGPRs: a wave-uniform value computed along paths
 // the divergence analysis cannot prove uniform would otherwise reach the
@@ -201,12 +205,12 @@ __device__ __forceinline__ void dma16(const u32x4& rsrc, uint32_t lds_addr, uint
   const uint32_t l = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_addr);
   const uint32_t so = (uint32_t)__builtin_amdgcn_readfirstlane((int)soff);
   if constexpr (NT)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
                  :
                  : "s"(l), "v"(voff), "s"(r), "s"(so)
                  : "m0");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  :
                  : "s"(l), "v"(voff), "s"(r), "s"(so)
                  : "m0");
