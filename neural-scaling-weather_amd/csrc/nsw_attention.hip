@@ -885,8 +885,9 @@ __global__ __launch_bounds__(NW * 64, HD <= 32 ? 4 : 3) void attn_f32_mfma_kerne
 //     are added at the end.
 // KSTR: the four head dims of a K or V read lie in other banks (48 mod 64).
 // Bound by the softmax's VALU work.  400 windows of 324, 8 heads of 4: 630 us in
-// attn_scalar_kernel, 148 in the kernel above with 4 x 4 x 1 blocks, 123 here (of
-// 162 tokens: 43 / 39); 8 heads of 8: 197 / 185.
+// attn_scalar_kernel, 148 with these instructions in the chunks of the kernel above
+// (three query blocks a wave in registers), 123 here (of 162 tokens: 43 / 39); 8
+// heads of 8: 197 / 185.
 template <int HD, bool MT, int CKB>
 __global__ __launch_bounds__(256, 5) void attn_f32_narrow_kernel(AttnArgs a) {
   constexpr int ROWS = CKB * 16, NDB = HD / 4;

@@ -12,12 +12,13 @@ namespace nsw {
 // at most the share f0 of the slots is (between them linear).  The constants
 // are fits to measured times (M 648 - 129600, N 32 - 4096, K 32 - 2048, bias
 // epilogue, within ~15%); 256 x 256 stays unless a smaller tile is estimated 7%
-// faster, since its epilogues are the tuned ones.  Measured, us, 256 x 256 /
-// 128 x 128 / 64 x 128:
-//   bf16   648 x  512, K  128:  7.8 /  4.7 /  3.8    16200 x  192, K  768: 17.7 / 11.2 / 10.6
-//   bf16  8100 x 1024, K 1024: 24.8 / 20.5 / 27.6    64800 x  512, K  512: 41.1 / 46.4 / 55.4
-//   fp32   648 x  128, K  512: 41.0 / 22.2 / 17.2    16200 x  192, K  768: 57.3 / 35.0 / 33.8
-//   fp32 129600 x 128, K   32: 27.1 / 17.3 / 17.9    32400 x  512, K  512: 62.2 / 76.5 / 90.0
+// faster, since its epilogues are the tuned ones.  The row epilogues go by the same
+// constants: their pick was the fastest or within 10% of it at 22 sizes of both
+// dtypes.  Measured, us, 256 x 256 / 128 x 128 / 64 x 128, bias epilogue:
+//   bf16   648 x  128, K  512: 13.1 /  7.9 /  5.9    16200 x  192, K  768: 16.9 / 10.7 /  9.8
+//   bf16  8100 x 1024, K 1024: 22.6 / 18.4 / 25.7    64800 x  512, K  512: 36.2 / 43.6 / 52.7
+//   fp32   648 x  128, K  512: 45.9 / 25.5 / 19.9    16200 x  192, K  768: 71.6 / 43.4 / 40.2
+//   fp32  8100 x 1024, K 1024: 97.6 / 76.3 / 97.0    32400 x  512, K  512: 58.8 / 77.5 / 91.7
 struct TileCost {
   int64_t bm, bn;
   double slots, fa, fb, pa, pb, f0;

@@ -1,4 +1,4 @@
-// Helpers of the MFMA GEMM kernel (nsw_gemm.hip): epilogue / operand-fusion
+// Helpers of the MFMA GEMM kernel (nsw_gemm_kernel.h): epilogue / operand-fusion
 // identifiers, the epilogue argument block, the GELU forms and the LDS row
 // swizzle of the operand stages.
 #pragma once

@@ -2,6 +2,10 @@
 // the Swin block's epilogues fused in: main loops, epilogues and the launch.
 // Included by one source per dtype and tile size.
 //
+// Three tile sizes (nsw_gemm_tiles.h); this is the bf16 256 x 256 one, whose main
+// loop is mainloop_256 (the smaller ones: mainloop_ring; fp32: mainloop_split2 and
+// mainloop_split3).
+//
 // Workgroup tile 256 (m) x 256 (n), one workgroup of 8 wavefronts per CU
 // (two per SIMD, so that one wave's MFMAs cover the other's LDS reads and
 // waits) in a 2 (m) x 4 (n) grid, each owning a 128 x 64 sub-tile of 16x16
@@ -23,9 +27,9 @@
 // weight fragment of an n block is read into the registers that block's
 // MFMAs have just released, so the x fragments are double-buffered and the
 // w fragments take one set (the register file of two waves per SIMD has no
-// room for two of both).  Barriers are bare
-// s_barrier: __syncthreads() would add a fence that waits for every
-// outstanding copy.
+// room for two of both).  Barriers are s_barrier behind a wait for the
+// wave's own LDS accesses: __syncthreads() would add a fence that waits for
+// every outstanding copy.
 //
 // The MFMA is issued "transposed": the A operand is the weight fragment
 // (rows n) and the B operand the activation fragment (rows m), so lane l of a
