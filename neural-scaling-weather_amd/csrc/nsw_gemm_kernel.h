@@ -586,10 +586,19 @@ __device__ __forceinline__ void add_outside(const Split2List& list, const int* s
   const int frow = lane & 15, fg = lane >> 4;
   const int xw = (wave / TC::WGN) * TC::WTM, ww = (wave % TC::WGN) * TC::WTN;   // this wave's first x and w rows
   const int n = __builtin_amdgcn_readfirstlane(list.n < split2_list<TC> ? list.n : split2_list<TC>);
-#pragma unroll 1
+  // lane i has entry i and its place in the order of k and row: the order of the
+  // list is the waves', and sums are to repeat bit for bit
+  const int lrow = list.row[lane < n ? lane : 0], lk = list.k[lane < n ? lane : 0];
+  int place = 0;
   for (int i = 0; i < n; ++i) {
-    int row = __builtin_amdgcn_readfirstlane(list.row[i]);
-    const int k = __builtin_amdgcn_readfirstlane(list.k[i]);
+    const int r = __builtin_amdgcn_readlane(lrow, i), k = __builtin_amdgcn_readlane(lk, i);
+    place += k < lk || (k == lk && r < lrow);
+  }
+#pragma unroll 1
+  for (int t = 0; t < n; ++t) {
+    const int i = __builtin_ctzll(__ballot(lane < n && place == t));
+    int row = __builtin_amdgcn_readlane(lrow, i);
+    const int k = __builtin_amdgcn_readlane(lk, i);
     const bool one = row >= SPLIT2_ONE;
     row &= SPLIT2_ONE - 1;
     const bool isx = row < TC::BM;
@@ -620,8 +629,8 @@ __device__ __forceinline__ void add_outside(const Split2List& list, const int* s
       for (int j = 0; j < G; ++j) {
         const float os = scale(!isx, b + j);
         // the other unit may have values without parts itself
-        const int orow = isx ? TC::BM + ww + (b + j) * 16 : xw + (b + j) * 16, l = lane < n ? lane : 0;
-        const bool both = (one || !isx) && __ballot(lane < n && list.row[l] == orow && list.k[l] == k) != 0;
+        const int orow = isx ? TC::BM + ww + (b + j) * 16 : xw + (b + j) * 16;
+        const bool both = (one || !isx) && __ballot(lane < n && lrow == orow && lk == k) != 0;
         f32x4 c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < 8; ++e) {

@@ -209,6 +209,23 @@ def test_split_gemm_on_each_tile(case, M, N, rows, K):
     _check(x, w)
 
 
+@pytest.mark.parametrize("M,N", [(301, 264), (5000, 1160), (8100, 3080)])
+def test_listed_units_repeat_bit_for_bit(M, N):
+    """Several corrections meet in most results; their order is not the waves'."""
+    K = 512
+    g = torch.Generator(device=_dev()).manual_seed(10)
+    x = torch.randn(M, K, generator=g, device=_dev())
+    w = 0.02 * torch.randn(N, K, generator=g, device=_dev())
+    for i, k in enumerate((70, 200, 330, 460)):
+        x[i::64, k] = 1e6 * (i + 1)
+        w[i::128, k + 33] = 1e4 * (i + 1)
+        w[:, k], x[:, k + 33] = 1e-6 * w[:, k], 1e-4 * x[:, k + 33]
+    first = _linear(x, w)
+    _check(x, w)
+    for _ in range(6):
+        assert torch.equal(_linear(x, w), first)
+
+
 # Shapes on both sides of the tile rule (64- / 32-row tiles; at 8100 x 1024 rows
 # 128- / 64-row tiles; then 256), with rows and columns that end
 # inside a tile, odd k stages, and every kind of write-out: plain, GELU,
