@@ -516,7 +516,7 @@ constexpr int SPLIT2_ONE = 1 << 16;
 // 2^-25 short, so a result of its row at most 2^-25 SPLIT2_MAX < 2^-9 (all scaled).
 // Returns the entries (bits) with a result of this wave that is not 2^20 times what
 // the row's small values may take from it; what their parts are short of is to be
-// added (normal rows, K = 1024: 5e-4 of the entries and results' blocks).  Results
+// added (normal rows, K = 1024: about 4 entries in 1000).  Results
 // below 4 become NaN, which redo_nonfinite forms again: a product of a subnormal part
 // takes part in the instruction's alignment as if the part were 2^-14, which may
 // take 2^-22 from the others'.  Rows of x or of w that are zero throughout (sh:
@@ -674,14 +674,14 @@ __device__ __forceinline__ void add_outside(const Split2List& list, const int* s
 // The unit of one outside goes on a list.  A single small value keeps its parts;
 // the results of its row are looked at in the end, and what the parts are short of
 // is added where it matters (check_small, add_outside).  Otherwise the values
-// outside get zero parts and their products are added in the end.  A product keeps within (K / 8 + 4) 2^-24 of itself
-// whatever else its rows hold, a quarter of what K fp32 additions may lose: lo = 8 /
-// K costs each of the two values K / 16 2^-24, and leaving out the product of the l
-// parts 4 2^-24.  lo is no lower than 2^-6, so that a value is never further off
-// than 2^-19.  Rows of normal values put about 5 K / 1024 units of a 256 x 256 tile
-// on the list, nearly all with one small value.  A tile whose list is full leaves
-// the loop before the stage that did not fit; the caller goes on from that stage
-// (the return value) on three parts.
+// outside get zero parts and their products are added in the end.  A product keeps
+// within (K / 8 + 4) 2^-24 of itself whatever else its rows hold, a quarter of what
+// K fp32 additions may lose: lo = 8 / K costs each of the two values K / 16 2^-24,
+// and leaving out the product of the l parts 4 2^-24.  lo is no lower than 2^-6, so
+// that a value is never further off than 2^-19.  Rows of normal values put about 5 K
+// / 1024 units of a 256 x 256 tile on the list, nearly all with one small value.  A
+// tile whose list is full leaves the loop before the stage that did not fit; the
+// caller goes on from that stage (the return value) on three parts.
 //
 // A row's scale is set at its first stage that is not zero throughout
 // (split2_scale; until then it is 0).
