@@ -29,7 +29,8 @@
 // fp32 (attn_f32_mfma_kernel; head dims 4 and 8: attn_f32_narrow_kernel): any
 // mask, windows of up to 384 tokens, on the fp32 matrix instructions.
 //
-// Generic path (attn_scalar_kernel: larger windows, bf16 at other head dims):
+// Generic path (attn_scalar_kernel: windows of few tokens or more than 384, bf16 at
+// other head dims):
 // one thread per query, online softmax over 64-key chunks staged in LDS, fp32
 // throughout.
 #include "nsw_common.h"
@@ -1133,8 +1134,15 @@ static int launch_dma(const AttnArgs& a0, int64_t items, hipStream_t st) {
   return 0;
 }
 
-// fp32 MFMA attention.  Returns -1 when it does not apply: windows above 384
-// tokens, unaligned tensors, a scale that is not positive (the row maximum is
+// Tokens of a window from which the fp32 MFMA kernels are faster than
+// attn_scalar_kernel: they fill and multiply whole chunks of 96 or 176 keys.
+// Measured, us, scalar / MFMA, 128 channels, 32400 tokens, no mask: head dim 4, 4
+// tokens 393 / 410, 9 302 / 184; 16, 4 170 / 262, 9 135 / 123; 32, 4 148 / 357, 9
+// 118 / 167, 16 108 / 96; 64, 1 438 / 689, 4 197 / 171; 128, 1 851 / 338.
+static int f32_mfma_min_tokens(int hd) { return hd <= 8 ? 5 : hd == 16 ? 9 : hd == 32 ? 13 : hd == 64 ? 4 : 1; }
+
+// fp32 MFMA attention.  Returns -1 when it does not apply: windows of few or above
+// 384 tokens, unaligned tensors, a scale that is not positive (the row maximum is
 // taken of the raw products) or whose -100 / scale is not finite.
 template <int HD>
 static int launch_f32_mfma_hd(const AttnArgs& a, int64_t items, hipStream_t st) {
@@ -1163,7 +1171,7 @@ static int launch_f32_narrow(const AttnArgs& a, int64_t items, hipStream_t st) {
 }
 
 static int launch_f32_mfma(const AttnArgs& a0, int hd, int64_t items, hipStream_t st) {
-  if (a0.L > 384 || items >= (1ll << 31)) return -1;
+  if (a0.L < f32_mfma_min_tokens(hd) || a0.L > 384 || items >= (1ll << 31)) return -1;
   if ((uintptr_t)a0.qkv % 16 != 0 || (uintptr_t)a0.o % 16 != 0) return -1;
   AttnArgs a = a0;
   a.zscale = a.scale * 1.4426950408889634f;

@@ -41,6 +41,19 @@ def test_attention_f32_sizes(hd, heads, L, masked):
     assert _rel(o, _ref(qkv, heads, hd ** -0.5, mask)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
 
 
+# both sides of the line below which windows go to the generic kernel (4 to 13
+# tokens); the bound as above
+@pytest.mark.parametrize("hd,heads", [(4, 6), (8, 3), (16, 2), (32, 3), (64, 2), (128, 1)])
+@pytest.mark.parametrize("L", [3, 4, 5, 8, 9, 12, 13])
+def test_attention_f32_few_tokens(hd, heads, L):
+    qkv = _qkv(6, L, hd * heads, L)
+    g = torch.Generator(device="cuda:0").manual_seed(L)
+    mask = torch.randn(2, L, L, generator=g, device="cuda:0")
+    for m in (None, mask):
+        o = nsw.ops.window_attention(qkv, heads, hd ** -0.5, mask=m)
+        assert _rel(o, _ref(qkv, heads, hd ** -0.5, m)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
+
+
 @pytest.mark.parametrize("L", [100, 324])
 def test_attention_f32_mask_extremes(L):
     """Keys masked with -inf (a whole leading chunk of them too), rows masked with
