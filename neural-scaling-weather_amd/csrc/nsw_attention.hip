@@ -1147,7 +1147,14 @@ static int f32_mfma_min_tokens(int hd) { return hd <= 8 ? 5 : hd == 16 ? 9 : hd 
 template <int HD>
 static int launch_f32_mfma_hd(const AttnArgs& a, int64_t items, hipStream_t st) {
   const bool mt = a.mask_mode == MASK_TENSOR;
-  if (a.L <= 192) {
+  // Eight waves a (window, head) for windows that four do not hold, and for those of
+  // more than four query blocks while the items do not fill the CUs more than once.
+  // Four / eight waves, us, 162 tokens, no mask, 8 | 256 | 400 items: head dim 16
+  // 10.8 / 9.2 | 11.9 / 10.1 | 17.1 / 15.8; 32 16.7 / 13.2 | 18.7 / 15.2 | 27.5 / 24.9;
+  // 64 28.3 / 23.3 | 33.1 / 27.9 | 49.2 / 47.2 (with a mask tensor 53.5 / 57.6);
+  // 128 57.6 / 44.4 | 69.0 / 54.5 | 97.2 / 98.4.
+  const bool four = a.L <= 64 || (a.L <= 192 && items > 256);
+  if (four) {
     if (mt) hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 4, true>), dim3((unsigned)items), dim3(256), 0, st, a);
     else hipLaunchKernelGGL((attn_f32_mfma_kernel<HD, 4, false>), dim3((unsigned)items), dim3(256), 0, st, a);
   } else {

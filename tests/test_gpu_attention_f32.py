@@ -54,6 +54,19 @@ def test_attention_f32_few_tokens(hd, heads, L):
         assert _rel(o, _ref(qkv, heads, hd ** -0.5, m)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
 
 
+# more items than CUs (four waves an item up to 192 tokens; fewer items above take
+# eight up from 65 tokens); the bound as above
+@pytest.mark.parametrize("hd", [16, 32, 64, 128])
+@pytest.mark.parametrize("L", [64, 65, 96, 162, 192])
+@pytest.mark.parametrize("items", [256, 258])
+def test_attention_f32_wave_counts(hd, L, items):
+    qkv = _qkv(items // 2, L, 2 * hd, L)
+    g = torch.Generator(device="cuda:0").manual_seed(L)
+    for mask in (None, torch.randn(1, L, L, generator=g, device="cuda:0")):
+        o = nsw.ops.window_attention(qkv, 2, hd ** -0.5, mask=mask)
+        assert _rel(o, _ref(qkv, 2, hd ** -0.5, mask)) < 2.0 ** -24 * (hd + 2 * L ** 0.5 + 8)
+
+
 @pytest.mark.parametrize("L", [100, 324])
 def test_attention_f32_mask_extremes(L):
     """Keys masked with -inf (a whole leading chunk of them too), rows masked with
